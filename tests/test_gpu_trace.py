@@ -119,6 +119,37 @@ def test_edge_cases(c1, oracle, gpu_ctx_factory):
             _assert_hits_equal(ctx.trace_closest(o, d, t), osc.trace_closest(o, d, t), osc, o, d, t)
 
 
+@pytest.mark.parametrize("stack_lds,block", [(8, 64), (8, 256), (16, 128), (16, 256), (32, 256)])
+@pytest.mark.parametrize("instanced", [False, True])
+def test_deep_stacks(stack_lds, block, instanced, oracle, gpu_ctx_factory):
+    """20000 stacked sheets: a ray along the pile meets every box of the
+    tree, so each level leaves three entries on the stack and it runs past
+    the LDS rows of every tuned depth but the largest; max_t from far below
+    zero to infinity."""
+    n = 20000
+    tris = np.zeros(n, scenes.TRI)
+    z = (np.arange(n) * 0.01).astype(np.float32)
+    for k, (x, y) in zip("abc", [(-4, -4), (4, -4), (0, 5)]):
+        tris[k][:, 0], tris[k][:, 1], tris[k][:, 2] = x, y, z
+        tris["n" + k][:, 2] = 1
+    sc = scenes.Scene(tris, scenes.lambert((0.5, 0.5, 0.5)), None, None, None)
+    if instanced:
+        sc.meshes = [tris[::50].copy()]
+        sc.instances = np.concatenate([scenes.make_instance(np.eye(3) * 0.5, (0.1 * i, 0, 0.003), 0) for i in range(9)])
+    rng = np.random.default_rng(3)
+    m = 3001
+    o = np.stack([rng.uniform(-1, 1, m), rng.uniform(-1, 1, m), rng.uniform(-20, 220, m)], 1).astype(np.float32)
+    d = rng.normal(scale=[0.02, 0.02, 1.0], size=(m, 3)).astype(np.float32)
+    t = rng.choice(np.float32([FMAX, np.inf, 60.0, 0.004, 0.0, -0.5, -1.0, -3.0, -FMAX, -np.inf]), m)
+    osc = oracle.OracleScene(tris, meshes=sc.meshes, instances=sc.instances)
+    with gpu_ctx_factory() as ctx:
+        ctx.set_tuning(stack_lds=stack_lds, trace_block=block)
+        ctx.upload(sc, max_leaf=1)
+        g, ref = ctx.trace_closest(o, d, t), osc.trace_closest(o, d, t)
+        assert (g == ref).all()
+        assert ((ctx.trace_any(o, d, t) != 0) == (ref["ref"] != 0xFFFFFFFF)).all()
+
+
 def test_call_order_and_argument_errors(c1, gpu_ctx_factory):
     with gpu_ctx_factory() as ctx:
         with pytest.raises(GiError) as e:
