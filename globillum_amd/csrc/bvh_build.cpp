@@ -595,41 +595,52 @@ void halton_permutation(int32_t dim, uint32_t seed, uint16_t *perm) {
   for (int32_t i = p - 1; i >= 1; --i) std::swap(perm[i], perm[r.bounded((uint32_t)(i + 1))]);
 }
 
-void halton_tables(uint32_t seed, int32_t ndims, std::vector<HaltonDim> &dims, std::vector<uint16_t> &chunks) {
+void halton_tables(uint32_t seed, int32_t ndims, std::vector<HaltonDim> &dims, std::vector<uint16_t> &perms,
+                   uint32_t &entries) {
   dims.resize(ndims);
-  chunks.clear();
-  std::vector<uint16_t> perm;
+  perms.clear();
+  entries = 0;
   for (int32_t d = 0; d < ndims; ++d) {
     const uint32_t p = (uint32_t)prime_of(d);
-    perm.resize(p);
-    halton_permutation(d, seed, perm.data());
-    uint32_t m = 1, P = p;
-    while (P * p <= 1024u) {
-      P *= p;
-      ++m;
-    }
     HaltonDim &h = dims[d];
     h.prime = p;
-    h.chunk_off = (uint32_t)chunks.size();
-    h.P = P;
-    h.perm0 = perm[0];
-    h.magic = (uint64_t)(~0ULL / P) + 1ULL;  // exact floor(n / P) = mulhi(n, magic) for n < 2^32
-    h.kmax = 0;
-    for (uint64_t pk = 1; pk < ((uint64_t)1 << 32); pk *= P) ++h.kmax;
-    h.pad = 0;
-    chunks.resize(chunks.size() + P);
-    for (uint32_t c = 0; c < P; ++c) {
-      uint32_t v = 0, x = c;
-      for (uint32_t i = 0; i < m; ++i) {  // least significant digit first
-        v = v * p + perm[x % p];
-        x /= p;
-      }
-      chunks[h.chunk_off + c] = (uint16_t)v;
+    h.perm_off = (uint32_t)perms.size();
+    perms.resize(perms.size() + p);
+    halton_permutation(d, seed, perms.data() + h.perm_off);
+    h.perm0 = perms[h.perm_off];
+    h.P = p;
+    h.m = 1;
+    while ((uint64_t)h.P * p <= 65536u) {
+      h.P *= p;
+      ++h.m;
     }
+    // two full chunks and a top chunk no longer than they, else three (from
+    // p = 257 on, where a chunk is one digit)
+    const uint64_t all = (uint64_t)1 << 32;
+    uint64_t pf = (uint64_t)h.P * h.P;
+    h.full = 2;
+    if (pf * h.P < all) {
+      pf *= h.P;
+      h.full = 3;
+    }
+    h.Ptop = 1;
+    h.mt = 0;
+    while (pf * h.Ptop < all) {
+      h.Ptop *= p;
+      ++h.mt;
+    }
+    h.off = entries;
+    h.top_off = h.off + h.P;
+    entries = h.top_off + h.Ptop;
+    h.magic = (uint64_t)(~0ULL / h.P) + 1ULL;  // exact floor(n / P) = mulhi(n, magic) for n < 2^32
+    h.p1 = (double)(p - 1);
+    h.perm0d = (double)h.perm0;
+    h.c_hi = (double)((uint64_t)(h.full == 3 ? h.P : 1u) * h.Ptop * (p - 1));
+    h.B = (double)(pf * h.Ptop * (p - 1));
+    h.rB = 1.0 / h.B;
   }
 }
 
-// Scrambled radical inverse as the exact rational A/B (see gi_device.h).
 float halton_host(uint64_t n, int32_t dim, uint32_t seed) {
   const int32_t p = prime_of(dim);
   std::vector<uint16_t> perm(p);

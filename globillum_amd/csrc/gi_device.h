@@ -122,80 +122,81 @@ __device__ __forceinline__ float cdf_sample(const float *__restrict__ cdf, const
 }
 
 // ---------------------------------------------------------------- Halton --
-// chunks holds the chunk tables from entry chunk_base of the pool on (0: the
-// whole pool in global memory; an LDS copy of some dimensions' tables starts
-// at the first one's offset)
 struct HaltonDev {
   const HaltonDim *dims;
-  const uint16_t *chunks;
-  uint32_t chunk_base;
+  const uint16_t *chunks;  // the chunk tables
 };
+// Chunk table entry c of dimension hd (the top chunk's table: c - P of the
+// entries past the full chunks').
+__device__ __forceinline__ uint16_t halton_entry(const HaltonDim &hd, const uint16_t *__restrict__ perms, uint32_t c) {
+  const bool top = c >= hd.P;
+  uint32_t x = top ? c - hd.P : c, v = 0;
+  const uint32_t m = top ? hd.mt : hd.m;
+  for (uint32_t i = 0; i < m; ++i) {  // least significant digit first
+    const uint32_t q = x / hd.prime;
+    v = v * hd.prime + perms[hd.perm_off + (x - q * hd.prime)];
+    x = q;
+  }
+  return (uint16_t)v;
+}
+// The chunk tables of dimension blockIdx.y.
+__global__ void __launch_bounds__(256) halton_fill(const HaltonDim *__restrict__ dims,
+                                                   const uint16_t *__restrict__ perms,
+                                                   uint16_t *__restrict__ chunks) {
+  const HaltonDim hd = dims[blockIdx.y];
+  for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < hd.P + hd.Ptop; c += gridDim.x * blockDim.x)
+    chunks[hd.off + c] = halton_entry(hd, perms, c);
+}
+
+typedef __attribute__((address_space(4))) HaltonDim HaltonDimConst;
 // Scrambled radical inverse of n in the prime base p of dimension dim: the
 // digits d_k (K of them) map to perm[d_k] and the infinitely many leading
 // zeros to perm[0], which is the exact rational
 //   A / B,  A = rev*(p-1) + perm[0],  B = p^K (p-1),  rev = sum perm[d_k] p^(K-1-k).
-// Digits are consumed m at a time through the chunk table (P = p^m <= 1024).
 // Leading zero digits may be counted as digits: each adds perm[0] to rev and
 // a factor p to p^K, which multiplies A and B by p and leaves A / B as it
-// is.  So every n is split into the same kmax chunks of its dimension (the
-// least K with P^K >= 2^32), zero chunks above its leading one included:
-// A, B <= 2^42 p stay exact in FP64 (every partial value is an integer below
-// 2^53), and the value is one correctly rounded FP64 division and one
-// rounding to FP32, as if only n's own digits were used.  kmax is the same
-// for every lane, so the chunks are taken with no per-lane selection.
-// floor(m / P) is the top 32 bits of the 96-bit m * magic (one 32-bit
-// mulhi and one 32x32+32 multiply-add: exact as the 64-bit mulhi); no
-// 64-bit integer multiplies, the quarter-rate part of this function.
-constexpr int kHaltonMaxChunks = 7;  // kmax <= 7: every dimension has P >= 37
+// is.  So every n < 2^32 is split into the same chunks of its dimension
+// (HaltonDim), and A, B < 2^32 p^2 are exact in FP64 (integers below 2^53).
+// The value is RN32(RN64(A / B)): with rB = RN(1/B) and q = RN(A rB), one
+// fused residual and one fused correction give the correctly rounded
+// quotient (Markstein, IBM J. Res. Dev. 34(1), 1990), three instructions in
+// place of the FP64 division's twenty.
+// Its quarter-rate integer products are the two of n / P (the top 32 bits
+// of the 96-bit n * magic; exact as the 64-bit mulhi) and one of the second
+// quotient: for q < 2^32 / P, floor(q / P) = mulhi(q, floor(2^32 / P) + 1),
+// since q times the multiplier's excess (<= P / 2^32) stays below 1 / P.
+// A sample's chunks are two of up to 65536 values and a top one (seven of up
+// to 1024, read from an LDS copy, before): the indices of a wave are mostly
+// consecutive, so its table reads fall into one or two lines (the low chunk)
+// or one entry (the others).  The shading kernels issue 22 % fewer vector
+// instructions with it and take 7.4 instead of 8.7 ms of the ~300k-triangle
+// frame and 85 instead of 97 ms of the 4.2M-triangle textured one; what
+// bounds them now is memory latency at 4 waves per SIMD.
 __device__ __forceinline__ float halton(uint32_t n, int dim, HaltonDev H) {
-  const HaltonDim hd = H.dims[dim];
-  const uint16_t *chunk = H.chunks + (hd.chunk_off - H.chunk_base);
-  const uint32_t mlo = (uint32_t)hd.magic, mhi = (uint32_t)(hd.magic >> 32);
-  uint32_t c[kHaltonMaxChunks];
-  uint32_t m = n;
-#pragma unroll
-  for (int k = 0; k < kHaltonMaxChunks; ++k) {
-    // (m * mhi + hi32(m * mlo)) >> 32 = hi64(m * magic): the low word of
-    // m * mlo cannot carry into the top 32 bits of the 96-bit product
-    const uint32_t q = (uint32_t)(((uint64_t)m * mhi + __umulhi(m, mlo)) >> 32);
-    c[k] = m - q * hd.P;
-    m = q;
+  // read through the constant address space: the dimension is the same for
+  // every lane of a kernel's wave, so these are scalar loads (plain loads
+  // would be vector loads, repeated after every store)
+  const HaltonDimConst &hd = ((const HaltonDimConst *)H.dims)[dim];
+  const uint16_t *tab = H.chunks + hd.off, *top = H.chunks + hd.top_off;
+  const uint32_t P = hd.P, mlo = (uint32_t)hd.magic, mhi = (uint32_t)(hd.magic >> 32);
+  // (n * mhi + hi32(n * mlo)) >> 32 = hi64(n * magic): the low word of
+  // n * mlo cannot carry into the top 32 bits of the 96-bit product
+  const uint32_t q0 = (uint32_t)(((uint64_t)n * mhi + __umulhi(n, mlo)) >> 32);
+  const uint32_t mq = mhi + 1u;  // floor(2^32 / P) + 1
+  const uint32_t q1 = __umulhi(q0, mq);
+  const uint32_t v0 = tab[n - __umul24(q0, P)], v1 = tab[q0 - __umul24(q1, P)];
+  uint32_t lo;
+  if (hd.full == 2) {  // uniform: one dimension per sample call
+    lo = top[q1];
+  } else {
+    const uint32_t q2 = __umulhi(q1, mq);
+    lo = __umul24(tab[q1 - __umul24(q2, P)], hd.Ptop) + top[q2];
   }
-  uint32_t v[kHaltonMaxChunks];
-#pragma unroll
-  for (int k = 0; k < kHaltonMaxChunks; ++k) v[k] = chunk[c[k]];
-  const double Pd = (double)hd.P;
-  double rev = 0.0, pk = 1.0;
-#pragma unroll
-  for (int k = 0; k < kHaltonMaxChunks; ++k) {
-    if ((uint32_t)k < hd.kmax) {
-      rev = fma(rev, Pd, (double)v[k]);
-      pk = pk * Pd;
-    }
-  }
-  const double p1 = (double)(hd.prime - 1);
-  const double A = fma(rev, p1, (double)hd.perm0), B = pk * p1;
-  const float f = (float)(A / B);
+  const uint32_t hi = __umul24(v0, P) + v1;
+  const double A = fma((double)hi, hd.c_hi, fma((double)lo, hd.p1, hd.perm0d));
+  const double q = A * hd.rB;
+  const float f = (float)fma(fma(-q, hd.B, A), hd.rB, q);
   return f >= 1.0f ? 0x1.fffffep-1f : f;
-}
-
-// The chunk tables of any kDimsPerVertex consecutive dimensions of a render
-// of depth <= 32 fit this many entries (the largest such window, dimensions
-// 221..227 with P = p from 1399 to 1439, holds 9959); the host checks it.
-constexpr uint32_t kHaltonLdsEntries = 10240;
-// Copies the chunk tables of dimensions [d0, d0 + nd) into lds and returns
-// the sampler that reads them there: the same values, with LDS reads in
-// place of the scattered 16-bit global loads.  Called by every thread of
-// the block, before any of them samples.  (The copy is addressed from its
-// own start, chunk_base = the first table's offset: a pointer moved below
-// the array would leave it, and in a flat address the borrow is lost.)
-__device__ __forceinline__ HaltonDev halton_in_lds(HaltonDev H, int d0, int nd, uint16_t *lds) {
-  const HaltonDim first = H.dims[d0], last = H.dims[d0 + nd - 1];
-  const uint32_t off0 = first.chunk_off - H.chunk_base;
-  const uint32_t n = min(last.chunk_off + last.P - first.chunk_off, kHaltonLdsEntries);
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) lds[i] = H.chunks[off0 + i];
-  __syncthreads();
-  return HaltonDev{H.dims, lds, first.chunk_off};
 }
 
 // ---------------------------------------------------------- frames -------

@@ -137,24 +137,34 @@ constexpr uint32_t kMaxInstances = kMaxLeafFirst - 2;
 
 // ------------------------------------------------------------- Halton ----
 // Per-dimension constants of the scrambled radical inverse, laid out for
-// the device.  Digits are consumed m at a time (P = p^m <= 1024): chunk[c]
-// for c < P holds the scrambled, reversed m-digit value
-// sum_i perm[digit_i(c)] p^(m-1-i); magic = floor(2^64/P)+1 divides by P.
+// the device.  An index n < 2^32 is split, lowest digits first, into `full`
+// chunks of m digits (P = p^m, the largest <= 65536) and a top chunk of mt
+// digits (Ptop = p^mt): P^full * Ptop >= 2^32.  Entry c of a chunk table is
+// the scrambled reversed value sum_i perm[digit_i(c)] p^(m-1-i) of the m
+// digits of c: below P, so 16 bits hold it.
 struct HaltonDim {
   uint32_t prime;       // p
-  uint32_t chunk_off;   // offset of the chunk table in the uint16 pool
-  uint32_t P;           // p^m
+  uint32_t off;         // the table of the full chunks in the uint16 pool
+  uint32_t top_off;     // the table of the top chunk
+  uint32_t perm_off;    // perm in the pool of digit permutations
+  uint32_t P, Ptop;
+  uint32_t full;        // full chunks: 2 or 3
+  uint32_t m, mt;       // digits of a full chunk and of the top chunk
   uint32_t perm0;       // perm[0]
   uint64_t magic;       // floor(2^64 / P) + 1
-  uint32_t kmax;        // chunks of any n < 2^32: the least K with P^K >= 2^32
-  uint32_t pad;
+  // A = hi * c_hi + lo * (p - 1) + perm[0], B = P^full Ptop (p - 1), 1 / B:
+  // integers below 2^53 (but for the last)
+  double c_hi, p1, perm0d, B, rB;
 };
-static_assert(sizeof(HaltonDim) == 32, "halton dim layout");
+static_assert(sizeof(HaltonDim) == 88, "halton dim layout");
 
 int32_t prime_of(int32_t dim);
 void halton_permutation(int32_t dim, uint32_t seed, uint16_t *perm);
-void halton_tables(uint32_t seed, int32_t ndims, std::vector<HaltonDim> &dims,
-                   std::vector<uint16_t> &chunks);
+// The dimensions' constants, the digit permutations they index and the
+// number of chunk table entries (which halton_fill of gi_device.h computes
+// on the device, one after another).
+void halton_tables(uint32_t seed, int32_t ndims, std::vector<HaltonDim> &dims, std::vector<uint16_t> &perms,
+                   uint32_t &entries);
 float halton_host(uint64_t n, int32_t dim, uint32_t seed);
 
 // Sample dimension map: jitter x/y, lens x/y, then per path vertex b:

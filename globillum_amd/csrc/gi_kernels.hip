@@ -958,8 +958,6 @@ __global__ __launch_bounds__(256) void k_raygen(const PassDesc *__restrict__ pas
                                                 HaltonDev H, float4 *__restrict__ ray_o, float4 *__restrict__ ray_d,
                                                 float4 *__restrict__ path_l, float4 *__restrict__ rec,
                                                 uint32_t rec_stride, int32_t depth) {
-  __shared__ uint16_t s_halton[kHaltonLdsEntries];
-  H = halton_in_lds(H, kDimJitterX, kDimVertex0, s_halton);
   const uint32_t total = pass->total_slots;
   for (uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x; slot < total; slot += gridDim.x * blockDim.x) {
     const PassChunk &ck = pass->chunk[find_chunk(pass, slot)];
@@ -975,8 +973,12 @@ __global__ __launch_bounds__(256) void k_raygen(const PassDesc *__restrict__ pas
     // jittered (setup_jittered_shirley / _dof_shirley) or through the pixel
     // centre (setup_shirley_lens_rays, src/dofrays.cu:21-22)
     const float jx = v.centre ? 0.5f : halton(n, kDimJitterX, H), jy = v.centre ? 0.5f : halton(n, kDimJitterY, H);
-    camera_ray(v, (int32_t)(p % (uint32_t)v.w), (int32_t)(p / (uint32_t)v.w), jx, jy, halton(n, kDimLensX, H),
-               halton(n, kDimLensY, H), o, d);
+    float lx = 0.f, ly = 0.f;  // the lens sample, where there is a lens
+    if (v.aperture > 0.0f) {
+      lx = halton(n, kDimLensX, H);
+      ly = halton(n, kDimLensY, H);
+    }
+    camera_ray(v, (int32_t)(p % (uint32_t)v.w), (int32_t)(p / (uint32_t)v.w), jx, jy, lx, ly, o, d);
     ray_o[slot] = make_float4(o.x, o.y, o.z, bitsf(n));
     ray_d[slot] = make_float4(d.x, d.y, d.z, bitsf(slot));
     path_l[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1149,7 +1151,6 @@ __device__ __forceinline__ void phong_vertex(const ShadeParams &P, HaltonDev H, 
 }
 
 template <bool kTex, bool kPhong = false>
-// H: the sampler (its tables in global memory or an LDS copy)
 __device__ __forceinline__ void eval_vertex(const ShadeParams &P, HaltonDev H, uint32_t n, int dim, uint32_t slot,
                                             f3 org_dir, float4 h, VertexEval &ve) {
   uint32_t tid = fbits(h.w);
@@ -1337,11 +1338,7 @@ __device__ __forceinline__ void shade_vertices(
     uint32_t *__restrict__ next_count, float4 *__restrict__ sho, float4 *__restrict__ shd, float4 *__restrict__ shc,
     uint32_t *__restrict__ shadow_count, float4 *__restrict__ rec, uint32_t rec_stride) {
   const int dim = kDimVertex0 + kDimsPerVertex * b;
-  // the vertex's sample dimensions, read from an LDS copy of their tables;
-  // the textured kernel keeps reading them from global memory: with the LDS
-  // reads its schedule spills 11 registers instead of 2 and runs 5 % slower
-  __shared__ uint16_t s_halton[kHaltonLdsEntries];
-  const HaltonDev H = kTex ? P.H : halton_in_lds(P.H, dim, kDimsPerVertex, s_halton);
+  const HaltonDev H = P.H;
   const uint32_t count = *count_ptr;
   const bool last = b + 1 >= P.depth;
   for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += gridDim.x * blockDim.x) {
@@ -1433,9 +1430,7 @@ __device__ __forceinline__ void shade_vertices(
 }
 
 // Both shading kernels are held to 4 waves per SIMD (128 VGPRs): the
-// untextured one fits without spilling, the textured one spills two
-// registers; at the compiler's own choice they take 137 and 177
-// VGPRs (3 waves), which measured slower.
+// untextured one takes 95, the textured one spills two registers.
 #define GI_SHADE_ARGS                                                                                              \
   int32_t b, const uint32_t *__restrict__ count_ptr, ShadeParams P, const float4 *__restrict__ ray_o,             \
       const float4 *__restrict__ ray_d, const float4 *__restrict__ tp_in, const float4 *__restrict__ hits,        \
@@ -2152,22 +2147,20 @@ DevMatGrad make_devmatgrad(const gi_material &m) {
 int ensure_halton(gi_ctx *ctx, uint32_t seed, int32_t ndims) {
   if (ctx->hal_dims >= ndims && ctx->hal_seed == seed && ctx->d_hdims.p) return GI_OK;
   std::vector<HaltonDim> dims;
-  std::vector<uint16_t> perms;  // chunk tables
-  halton_tables(seed, ndims, dims, perms);
-  // ray generation and each shading launch copy the tables of their
-  // dimensions into LDS: kDimVertex0, then kDimsPerVertex at a time
-  for (int32_t d0 = 0; d0 < ndims;) {
-    const int32_t nd = std::min(d0 == 0 ? kDimVertex0 : kDimsPerVertex, ndims - d0);
-    if (dims[d0 + nd - 1].chunk_off + dims[d0 + nd - 1].P - dims[d0].chunk_off > kHaltonLdsEntries)
-      return fail(ctx, GI_ERR_LIMIT,
-                  "sampler tables of dimensions " + std::to_string(d0) + ".." + std::to_string(d0 + nd - 1) +
-                      " exceed the LDS copy");
-    d0 += nd;
-  }
+  std::vector<uint16_t> perms;
+  uint32_t entries = 0;
+  halton_tables(seed, ndims, dims, perms, entries);
+  DBuf d_perms;
+  GI_HIP(ctx, d_perms.ensure(perms.size() * sizeof(uint16_t)));
   GI_HIP(ctx, ctx->d_hdims.ensure(dims.size() * sizeof(HaltonDim)));
-  GI_HIP(ctx, ctx->d_hchunks.ensure(perms.size() * sizeof(uint16_t)));
+  GI_HIP(ctx, ctx->d_hchunks.ensure(entries * sizeof(uint16_t)));
+  ctx->hal_dims = 0;  // the old tables are gone from here on
   GI_HIP(ctx, copy_sync(ctx, ctx->d_hdims.p, dims.data(), dims.size() * sizeof(HaltonDim), hipMemcpyHostToDevice));
-  GI_HIP(ctx, copy_sync(ctx, ctx->d_hchunks.p, perms.data(), perms.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  GI_HIP(ctx, copy_sync(ctx, d_perms.p, perms.data(), perms.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(halton_fill, dim3(64, (uint32_t)ndims), dim3(256), 0, ctx->stream, ctx->d_hdims.as<HaltonDim>(),
+                     d_perms.as<uint16_t>(), ctx->d_hchunks.as<uint16_t>());
+  GI_HIP(ctx, hipGetLastError());
+  GI_HIP(ctx, hipStreamSynchronize(ctx->stream));
   ctx->hal_seed = seed;
   ctx->hal_dims = ndims;
   return GI_OK;
@@ -2658,7 +2651,7 @@ ShadeParams shade_params(gi_ctx *ctx, int32_t depth) {
   P.lights = ctx->d_lights.as<DevLight>();
   P.nlights = (int32_t)ctx->lights.size();
   P.power_total = ctx->power_total;
-  P.H = HaltonDev{ctx->d_hdims.as<HaltonDim>(), ctx->d_hchunks.as<uint16_t>(), 0u};
+  P.H = HaltonDev{ctx->d_hdims.as<HaltonDim>(), ctx->d_hchunks.as<uint16_t>()};
   P.off_b = ctx->opts.offset_bounce > 0.f ? ctx->opts.offset_bounce : 1e-4f * ctx->diag;
   P.off_s = ctx->opts.offset_shadow > 0.f ? ctx->opts.offset_shadow : 1e-4f * ctx->diag;
   for (int k = 0; k < 3; ++k) P.bg[k] = ctx->opts.background[k];
@@ -3874,7 +3867,7 @@ int gi_generate_camera_rays(gi_ctx *ctx, const gi_view *v, int32_t sample, uint3
   GI_HIP(ctx, copy_sync(ctx, ctx->d_cam_view.p, &dv, sizeof(dv), hipMemcpyHostToDevice));
   rc = ensure_workspace(ctx, npix);
   if (rc) return rc;
-  HaltonDev H{ctx->d_hdims.as<HaltonDim>(), ctx->d_hchunks.as<uint16_t>(), 0u};
+  HaltonDev H{ctx->d_hdims.as<HaltonDim>(), ctx->d_hchunks.as<uint16_t>()};
   hipLaunchKernelGGL(k_raygen, dim3((npix + 255) / 256), dim3(256), 0, ctx->stream, ctx->d_cam_pass.as<PassDesc>(),
                      ctx->d_cam_view.as<DevView>(), H, ctx->q_o[0].as<float4>(), ctx->q_d[0].as<float4>(),
                      ctx->path_l.as<float4>(), (float4 *)nullptr, 0u, 1);

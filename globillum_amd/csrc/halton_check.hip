@@ -57,20 +57,24 @@ int main(int argc, char **argv) {
   std::fclose(fi);
   const uint32_t count = (uint32_t)(pairs.size() / 2);
   std::vector<gi::HaltonDim> dims;
-  std::vector<uint16_t> chunks;
-  gi::halton_tables(seed, kDims, dims, chunks);
-  void *d_pairs = nullptr, *d_dims = nullptr, *d_chunks = nullptr, *d_out = nullptr;
+  std::vector<uint16_t> perms;
+  uint32_t entries = 0;
+  gi::halton_tables(seed, kDims, dims, perms, entries);
+  void *d_pairs = nullptr, *d_dims = nullptr, *d_perms = nullptr, *d_chunks = nullptr, *d_out = nullptr;
   const size_t nb = std::max<size_t>(1, count);
   if (!ok(hipMalloc(&d_pairs, nb * 2 * sizeof(uint32_t)), "hipMalloc") ||
       !ok(hipMalloc(&d_out, nb * sizeof(float)), "hipMalloc") ||
       !ok(hipMalloc(&d_dims, dims.size() * sizeof(gi::HaltonDim)), "hipMalloc") ||
-      !ok(hipMalloc(&d_chunks, chunks.size() * sizeof(uint16_t)), "hipMalloc"))
+      !ok(hipMalloc(&d_perms, perms.size() * sizeof(uint16_t)), "hipMalloc") ||
+      !ok(hipMalloc(&d_chunks, entries * sizeof(uint16_t)), "hipMalloc"))
     return 2;
   if (!ok(hipMemcpy(d_pairs, pairs.data(), pairs.size() * sizeof(uint32_t), hipMemcpyHostToDevice), "copy") ||
       !ok(hipMemcpy(d_dims, dims.data(), dims.size() * sizeof(gi::HaltonDim), hipMemcpyHostToDevice), "copy") ||
-      !ok(hipMemcpy(d_chunks, chunks.data(), chunks.size() * sizeof(uint16_t), hipMemcpyHostToDevice), "copy"))
+      !ok(hipMemcpy(d_perms, perms.data(), perms.size() * sizeof(uint16_t), hipMemcpyHostToDevice), "copy"))
     return 2;
-  const gi::dev::HaltonDev H{static_cast<const gi::HaltonDim *>(d_dims), static_cast<const uint16_t *>(d_chunks), 0u};
+  hipLaunchKernelGGL(gi::dev::halton_fill, dim3(64, kDims), dim3(256), 0, 0, static_cast<const gi::HaltonDim *>(d_dims),
+                     static_cast<const uint16_t *>(d_perms), static_cast<uint16_t *>(d_chunks));
+  const gi::dev::HaltonDev H{static_cast<const gi::HaltonDim *>(d_dims), static_cast<const uint16_t *>(d_chunks)};
   if (count > 0)
     hipLaunchKernelGGL(k_halton_eval, dim3((count + 255) / 256), dim3(256), 0, 0,
                        static_cast<const uint32_t *>(d_pairs), count, H, static_cast<float *>(d_out));
@@ -88,6 +92,7 @@ int main(int argc, char **argv) {
   (void)hipFree(d_pairs);
   (void)hipFree(d_out);
   (void)hipFree(d_dims);
+  (void)hipFree(d_perms);
   (void)hipFree(d_chunks);
   std::printf("%u values\n", count);
   return 0;
