@@ -137,12 +137,75 @@ struct ShadeParams {
 __device__ __forceinline__ uint32_t fbits(float f) { return __float_as_uint(f); }
 __device__ __forceinline__ float bitsf(uint32_t u) { return __uint_as_float(u); }
 
-// Append of two predicates per thread across the whole block: one atomic
-// per counter per block (device-wide atomics on one address serialise, so
-// they are kept few).  Called uniformly by every thread of the block;
-// blockDim <= 256.
-__device__ __forceinline__ void block_append2(bool p0, uint32_t *c0, bool p1, uint32_t *c1, uint32_t &q0,
-                                              uint32_t &q1) {
+// ------------------------------------------------------------- queues ----
+// A ray queue is kShards segments of `cap` entries, segment k holding
+// entries [k cap, k cap + n_k).  A shading tile (blockDim consecutive inputs)
+// appends to the segment its inputs come from, or, for tile j of the path
+// slots, to segment (j / kShards) % kShards; a segment's counters lie in a
+// cache line of their own: one 64-bit atomic per tile (low word the next bounce's
+// rays, high word the shadow rays; the low count stays below 2^32, so it
+// never carries).  Device-wide atomics on one address serialise beyond the
+// L2s, and one counter pair per queue bounded the shading of small scenes:
+// with four, and 64 instead of 8 blocks per CU, the 16 Cornell views' shading
+// takes 42 instead of 57 ms, the 256x256 Cornell frame's 0.16 instead of
+// 0.22 ms and the 291k-triangle frame's 6.6 instead of 7.4 ms.  8 or 16
+// segments shade no faster and cost the traversal 1-2 % in order.
+// Consumers take spans or tiles j = 0, 1, 2, ...: kShards consecutive ones
+// from a segment, then as many from the next one, and so on round the
+// segments.  Tiles that lie side by side thus stay so, from bounce to bounce
+// (one tile per segment in turn, with 16 segments, put tiles 16 apart side by
+// side: the 4.2M-triangle frame's any-hit kernel took 96 instead of 93 ms).  shift 0 is
+// a queue of one segment (a pass's path slots, the primitive entry points'
+// rays).
+constexpr uint32_t kShardShift = 2, kShards = 1u << kShardShift;
+constexpr uint32_t kCountStride = 16;  // 32-bit words between the counter pairs of two segments
+typedef __attribute__((address_space(4))) uint32_t const_u32;
+struct QueueIn {
+  const uint32_t *counts;  // n_k at counts[k * kCountStride], or null: one segment of n_host
+  uint32_t n_host, shift, cap;
+  // span or tile j: its segment, its row there, and the least row of the
+  // spans or tiles from j on.  The segment is turned by j / 2048, so that a
+  // wave that takes every 6144th span meets all segments: some are longer
+  // than others (unturned, the 291k-triangle frame's traversal took 2 % more)
+  __device__ __forceinline__ void locate(uint32_t j, uint32_t &k, uint32_t &row, uint32_t &least) const {
+    k = shift ? ((j >> kShardShift) + (j >> 11)) & (kShards - 1u) : 0u;
+    least = shift ? (j >> (2u * kShardShift)) << kShardShift : j;
+    row = shift ? least | (j & (kShards - 1u)) : j;
+  }
+  // entries of segment k (scalar loads: written by an earlier kernel)
+  __device__ __forceinline__ uint32_t size(uint32_t k) const {
+    return counts ? ((const const_u32 *)counts)[k * kCountStride] : n_host;
+  }
+  __device__ __forceinline__ uint32_t longest(uint32_t &total) const {
+    uint32_t m = size(0);
+    total = m;
+    if (shift)
+#pragma unroll
+      for (uint32_t k = 1; k < kShards; ++k) {
+        const uint32_t n = size(k);
+        m = n > m ? n : m;
+        total += n;
+      }
+    return m;
+  }
+};
+// The counters of a pass (32-bit words): word 0 the path slots, then per
+// bounce the pairs its shading appends to.
+__host__ __device__ constexpr int32_t count_words(int32_t depth) {
+  return (int32_t)kCountStride * (1 + depth * (int32_t)kShards);
+}
+__host__ __device__ constexpr int32_t pair_word(int32_t b) { return (int32_t)kCountStride * (1 + b * (int32_t)kShards); }
+// Entries of a segment of the queues behind `slots` inputs in tiles of
+// `tile`: a tile appends at most one entry per input to each queue.
+__host__ __device__ constexpr uint32_t segment_cap(uint64_t slots, uint32_t tile) {
+  return (uint32_t)(((slots + tile - 1) / tile + kShards * kShards - 1) / (kShards * kShards) * kShards * tile);
+}
+
+// Append of two predicates per thread across the whole block to segment k:
+// positions q0, q1 in the queues.  Called uniformly by every
+// thread of the block; blockDim <= 256.
+__device__ __forceinline__ void block_append2(bool p0, bool p1, uint32_t k, uint32_t *pairs, uint32_t cap,
+                                              uint32_t &q0, uint32_t &q1) {
   __shared__ uint32_t s_n[2][4];
   __shared__ uint32_t s_base[2];
   const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
@@ -153,14 +216,22 @@ __device__ __forceinline__ void block_append2(bool p0, uint32_t *c0, bool p1, ui
     s_n[1][wave] = (uint32_t)__popcll(m1);
   }
   __syncthreads();
-  if (threadIdx.x < 2) {
-    const uint32_t k = threadIdx.x, nw = blockDim.x >> 6;
-    uint32_t tot = 0;
-    for (uint32_t w = 0; w < nw; ++w) tot += s_n[k][w];
-    s_base[k] = tot ? atomicAdd(k ? c1 : c0, tot) : 0u;
+  if (threadIdx.x == 0) {
+    const uint32_t nw = blockDim.x >> 6;
+    uint32_t t0 = 0, t1 = 0;
+    for (uint32_t w = 0; w < nw; ++w) {
+      t0 += s_n[0][w];
+      t1 += s_n[1][w];
+    }
+    unsigned long long base = 0;
+    if (t0 | t1)
+      base = atomicAdd(reinterpret_cast<unsigned long long *>(pairs + k * kCountStride),
+                       (unsigned long long)t1 << 32 | t0);
+    s_base[0] = (uint32_t)base;
+    s_base[1] = (uint32_t)(base >> 32);
   }
   __syncthreads();
-  uint32_t o0 = s_base[0], o1 = s_base[1];
+  uint32_t o0 = k * cap + s_base[0], o1 = k * cap + s_base[1];
   for (uint32_t w = 0; w < wave; ++w) {
     o0 += s_n[0][w];
     o1 += s_n[1][w];
@@ -387,7 +458,7 @@ __device__ __forceinline__ Stack<kRows, kDist> make_stack(uint32_t *smem, uint32
            (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u)), (int)cap};
 }
 
-// The persistent traversal loop over queue entries [0, count).
+// The persistent traversal loop over a queue's entries.
 //   start(i, o, d, tmax) loads ray i;
 //   finish(i, t, u, v, id) stores its result (id == GI_INVALID_REF: no hit).
 // kInst: two-level traversal from the instance tree's root.  An instance
@@ -408,7 +479,7 @@ __device__ __forceinline__ bool special_ref(uint32_t ref) {
 // kLdsScene: the block's LDS holds a copy of the f32 wide nodes (8 float4 each) at
 // lnodes and of the triangles at ltris; they are read from there.
 template <bool kAny, bool kInst, int kRows, bool kCount, bool kLdsScene, bool kDist, class Start, class Finish>
-__device__ __forceinline__ void trace_persistent(uint32_t count, uint32_t cs, const HalfNode *__restrict__ nodes,
+__device__ __forceinline__ void trace_persistent(QueueIn Q, uint32_t cs, const HalfNode *__restrict__ nodes,
                                                  const float4 *__restrict__ itris, const float4 *lnodes,
                                                  const float4 *ltris, Stack<kRows, kDist> &st, uint32_t *overflow,
                                                  InstScene IS, unsigned long long *stats, Start start,
@@ -419,17 +490,29 @@ __device__ __forceinline__ void trace_persistent(uint32_t count, uint32_t cs, co
   const uint32_t waves = gridDim.x * (blockDim.x >> 6);
   const uint32_t chunk_n = 1u << cs;  // idle lanes a refill needs
   // span length 2^ss (wave-uniform): 16 spans per wave at least, 256 rays at most
+  uint32_t total;
+  const uint32_t longest = Q.longest(total);
   uint32_t ss = cs;
-  while (ss < 8u && (((uint64_t)waves * 16u) << (ss + 1)) <= count) ++ss;
-  // the start and the end of span k, both clamped to count
-  const auto span_range = [&](uint32_t k, uint32_t &b, uint32_t &e) {
-    const uint64_t b64 = (uint64_t)k << ss;
-    b = b64 >= count ? count : (uint32_t)b64;
-    e = min(b + (1u << ss), count);
+  while (ss < 8u && (((uint64_t)waves * 16u) << (ss + 1)) <= total) ++ss;
+  // the first non-empty span of this wave from span j on (j moves to it),
+  // as queue entries [b, e); b == e: none is left
+  const uint32_t rows = (uint32_t)(((uint64_t)longest + (1u << ss) - 1) >> ss);
+  const auto span_from = [&](uint32_t &j, uint32_t &b, uint32_t &e) {
+    for (b = e = 0;; j += waves) {
+      uint32_t k, row, least;
+      Q.locate(j, k, row, least);
+      if (least >= rows) return;
+      const uint32_t n = Q.size(k), off = row << ss;
+      if (row < rows && off < n) {
+        b = k * Q.cap + off;
+        e = b + min(1u << ss, n - off);
+        return;
+      }
+    }
   };
-  uint32_t span = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);  // wave-uniform: current span
-  uint32_t cur, end;  // the wave's next ray, the end of its current span
-  span_range(span, cur, end);
+  uint32_t span = blockIdx.x * (blockDim.x >> 6) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  uint32_t cur, end;  // the wave's next ray, the end of its current span (cur == end: no ray is left)
+  span_from(span, cur, end);
   uint32_t ray = kNoRay, ref = kDoneRef, parked = kDoneRef;
   f3 o{0.f, 0.f, 0.f}, d{0.f, 0.f, 0.f}, idir{0.f, 0.f, 0.f}, oid{0.f, 0.f, 0.f};
   uint32_t neg = 0;  // dir_signs of the ray
@@ -442,10 +525,10 @@ __device__ __forceinline__ void trace_persistent(uint32_t count, uint32_t cs, co
     // the rest of its current span, then the start of its next one
     const uint64_t idle = __ballot(ray == kNoRay);
     const uint32_t n_idle = (uint32_t)__popcll(idle);
-    if (n_idle >= chunk_n && cur < count) {
+    if (n_idle >= chunk_n && cur < end) {
       const uint32_t rem = end - cur;  // >= 1
-      uint32_t nb, ne;
-      span_range(span + waves, nb, ne);
+      uint32_t next = span + waves, nb, ne;
+      span_from(next, nb, ne);
       const uint32_t n_take = min(n_idle, rem + (ne - nb));
       if (ray == kNoRay) {
         const uint32_t r = (uint32_t)__popcll(idle & below);
@@ -468,17 +551,17 @@ __device__ __forceinline__ void trace_persistent(uint32_t count, uint32_t cs, co
       if (n_take < rem) {
         cur += n_take;
       } else {
-        span += waves;
+        span = next;
         cur = nb + (n_take - rem);
         end = ne;
-        if (cur >= end) {
+        if (cur == end && nb < ne) {
           span += waves;
-          span_range(span, cur, end);
+          span_from(span, cur, end);
         }
       }
     }
     if (__ballot(ray != kNoRay) == 0) {
-      if (cur >= count) break;
+      if (cur == end) break;
       continue;
     }
     if (ray == kNoRay) continue;
@@ -773,19 +856,18 @@ __device__ __forceinline__ void stage_scene(uint32_t *smem, uint32_t stack_words
 
 template <bool kHasTmax, bool kInst, int kRows, bool kCount, bool kLdsScene>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GI_TRACE_WAVES_PER_EU))) void k_trace_closest(
-    const uint32_t *__restrict__ count_ptr, uint32_t count_host, const float4 *__restrict__ ray_o,
+    QueueIn Q, const float4 *__restrict__ ray_o,
     const float4 *__restrict__ ray_d, float4 *__restrict__ hits, const HalfNode *__restrict__ nodes,
     const WideNode *__restrict__ wnodes, const float4 *__restrict__ itris, uint32_t *__restrict__ gstack, uint32_t stack_cap, uint32_t *overflow,
     InstScene IS, unsigned long long *stats, uint32_t chunk_shift, uint32_t stack_words, uint32_t n_nodes,
     uint32_t n_tris) {
   extern __shared__ uint32_t smem[];
-  const uint32_t count = count_ptr ? *count_ptr : count_host;
   constexpr bool kDist = !kLdsScene;
   Stack<kRows, kDist> st = make_stack<kRows, kDist>(smem, gstack, stack_cap);
   const float4 *lnodes = nullptr, *ltris = nullptr;
   stage_scene<kLdsScene>(smem, stack_words, wnodes, n_nodes, itris, n_tris, lnodes, ltris);
   trace_persistent<false, kInst, kRows, kCount, kLdsScene, kDist>(
-      count, chunk_shift, nodes, itris, lnodes, ltris, st, overflow, IS, stats,
+      Q, chunk_shift, nodes, itris, lnodes, ltris, st, overflow, IS, stats,
       [&](uint32_t i, f3 &o, f3 &d, float &tmax) {
         const float4 ro = ray_o[i], rd = ray_d[i];
         o = xyz(ro);
@@ -801,7 +883,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GI_TRACE_WA
 // occlusion byte (primitive entry point).
 template <bool kDeposit, bool kInst, int kRows, bool kCount, bool kLdsScene>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GI_TRACE_WAVES_PER_EU))) void k_trace_any(
-    const uint32_t *__restrict__ count_ptr, uint32_t count_host, const float4 *__restrict__ ray_o,
+    QueueIn Q, const float4 *__restrict__ ray_o,
     const float4 *__restrict__ ray_d, const float4 *__restrict__ contrib, float4 *__restrict__ path_l,
     uint8_t *__restrict__ occluded, const HalfNode *__restrict__ nodes, const WideNode *__restrict__ wnodes,
     const float4 *__restrict__ itris,
@@ -809,12 +891,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GI_TRACE_WA
     uint32_t rec_stride, int32_t b, InstScene IS, unsigned long long *stats, uint32_t chunk_shift,
     uint32_t stack_words, uint32_t n_nodes, uint32_t n_tris) {
   extern __shared__ uint32_t smem[];
-  const uint32_t count = count_ptr ? *count_ptr : count_host;
   Stack<kRows, false> st = make_stack<kRows, false>(smem, gstack, stack_cap);
   const float4 *lnodes = nullptr, *ltris = nullptr;
   stage_scene<kLdsScene>(smem, stack_words, wnodes, n_nodes, itris, n_tris, lnodes, ltris);
   trace_persistent<true, kInst, kRows, kCount, kLdsScene, false>(
-      count, chunk_shift, nodes, itris, lnodes, ltris, st, overflow, IS, stats,
+      Q, chunk_shift, nodes, itris, lnodes, ltris, st, overflow, IS, stats,
       [&](uint32_t i, f3 &o, f3 &d, float &tmax) {
         const float4 ro = ray_o[i], rd = ray_d[i];
         o = xyz(ro);
@@ -1332,20 +1413,28 @@ constexpr uint32_t kRecBackground = 8u;
 // record the vertex for the adjoint (see kRecBackground).
 template <bool kTex, bool kPhong = false>
 __device__ __forceinline__ void shade_vertices(
-    int32_t b, const uint32_t *__restrict__ count_ptr, const ShadeParams &P, const float4 *__restrict__ ray_o,
+    int32_t b, const QueueIn &Q, const ShadeParams &P, const float4 *__restrict__ ray_o,
     const float4 *__restrict__ ray_d, const float4 *__restrict__ tp_in, const float4 *__restrict__ hits,
     float4 *__restrict__ path_l, float4 *__restrict__ nro, float4 *__restrict__ nrd, float4 *__restrict__ ntp,
-    uint32_t *__restrict__ next_count, float4 *__restrict__ sho, float4 *__restrict__ shd, float4 *__restrict__ shc,
-    uint32_t *__restrict__ shadow_count, float4 *__restrict__ rec, uint32_t rec_stride) {
+    uint32_t *__restrict__ pairs, uint32_t cap, float4 *__restrict__ sho, float4 *__restrict__ shd,
+    float4 *__restrict__ shc, float4 *__restrict__ rec, uint32_t rec_stride) {
   const int dim = kDimVertex0 + kDimsPerVertex * b;
   const HaltonDev H = P.H;
-  const uint32_t count = *count_ptr;
   const bool last = b + 1 >= P.depth;
-  for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += gridDim.x * blockDim.x) {
-    const uint32_t i = base + threadIdx.x;
+  uint32_t total;
+  const uint32_t longest = Q.longest(total);
+  for (uint32_t tile = blockIdx.x;; tile += gridDim.x) {
+    uint32_t k, row, least;
+    Q.locate(tile, k, row, least);
+    if ((uint64_t)least * blockDim.x >= longest) break;
+    const uint32_t off = row * blockDim.x, n_k = Q.size(k);
+    if (off >= n_k) continue;  // this segment is shorter
+    const uint32_t k_out = Q.shift ? k : (tile >> kShardShift) & (kShards - 1u);
+    const bool live = off + threadIdx.x < n_k;
+    const uint32_t i = k * Q.cap + off + threadIdx.x;
     bool emit_next = false, emit_shadow = false;
     float4 o_next, d_next, tp_next, s_o, s_d, s_c;
-    if (i < count) {
+    if (live) {
       const float4 ro = ray_o[i], rd = ray_d[i], h = hits[i];
       const float4 tpv = b == 0 ? make_float4(1.f, 1.f, 1.f, 0.f) : tp_in[i];  // a new path's throughput
       const uint32_t n = fbits(ro.w), slot = fbits(rd.w), id = fbits(h.w);
@@ -1415,7 +1504,7 @@ __device__ __forceinline__ void shade_vertices(
       }
     }
     uint32_t qn, qs;
-    block_append2(emit_next, next_count, emit_shadow, shadow_count, qn, qs);
+    block_append2(emit_next, emit_shadow, k_out, pairs, cap, qn, qs);
     if (emit_next) {
       nro[qn] = o_next;
       nrd[qn] = d_next;
@@ -1432,14 +1521,13 @@ __device__ __forceinline__ void shade_vertices(
 // Both shading kernels are held to 4 waves per SIMD (128 VGPRs): the
 // untextured one takes 95, the textured one spills two registers.
 #define GI_SHADE_ARGS                                                                                              \
-  int32_t b, const uint32_t *__restrict__ count_ptr, ShadeParams P, const float4 *__restrict__ ray_o,             \
-      const float4 *__restrict__ ray_d, const float4 *__restrict__ tp_in, const float4 *__restrict__ hits,        \
-      float4 *__restrict__ path_l, float4 *__restrict__ nro, float4 *__restrict__ nrd, float4 *__restrict__ ntp,  \
-      uint32_t *__restrict__ next_count, float4 *__restrict__ sho, float4 *__restrict__ shd,                      \
-      float4 *__restrict__ shc, uint32_t *__restrict__ shadow_count, float4 *__restrict__ rec, uint32_t rec_stride
-#define GI_SHADE_PASS                                                                                               \
-  b, count_ptr, P, ray_o, ray_d, tp_in, hits, path_l, nro, nrd, ntp, next_count, sho, shd, shc, shadow_count, rec, \
-      rec_stride
+  int32_t b, QueueIn Q, ShadeParams P, const float4 *__restrict__ ray_o, const float4 *__restrict__ ray_d,        \
+      const float4 *__restrict__ tp_in, const float4 *__restrict__ hits, float4 *__restrict__ path_l,             \
+      float4 *__restrict__ nro, float4 *__restrict__ nrd, float4 *__restrict__ ntp, uint32_t *__restrict__ pairs, \
+      uint32_t cap, float4 *__restrict__ sho, float4 *__restrict__ shd, float4 *__restrict__ shc,                 \
+      float4 *__restrict__ rec, uint32_t rec_stride
+#define GI_SHADE_PASS \
+  b, Q, P, ray_o, ray_d, tp_in, hits, path_l, nro, nrd, ntp, pairs, cap, sho, shd, shc, rec, rec_stride
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_shade(GI_SHADE_ARGS) {
   shade_vertices<false>(GI_SHADE_PASS);
 }
@@ -1646,28 +1734,36 @@ __device__ __forceinline__ void scatter_texel_grads(bool has, float *const ta[4]
 // dL/db * texel, and dL/db * colour goes to the four blended texels with
 // their bilinear weights (global atomics into the chain's gradient).
 template <bool kTex>
-__global__ __launch_bounds__(256) void k_shade_adjoint(int32_t b, const uint32_t *__restrict__ count_ptr,
+__global__ __launch_bounds__(256) void k_shade_adjoint(int32_t b, QueueIn Q,
                                                        ShadeParams P, AdjParams A, const float4 *__restrict__ ray_o,
                                                        const float4 *__restrict__ ray_d,
                                                        const float4 *__restrict__ tp_in, float4 *__restrict__ nro,
                                                        float4 *__restrict__ nrd, float4 *__restrict__ ntp,
-                                                       uint32_t *__restrict__ next_count) {
+                                                       uint32_t *__restrict__ pairs, uint32_t cap) {
   extern __shared__ float sg[];  // 5*nmats + 3*nlights
   const int ng = 5 * A.nmats + 3 * A.nlights;
   for (int k = threadIdx.x; k < ng; k += blockDim.x) sg[k] = 0.0f;
   __syncthreads();
-  const uint32_t count = *count_ptr;
   const int dim = kDimVertex0 + kDimsPerVertex * b;
   const bool last = b + 1 >= P.depth;
-  for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += gridDim.x * blockDim.x) {
-    const uint32_t i = base + threadIdx.x;
+  uint32_t total;
+  const uint32_t longest = Q.longest(total);
+  for (uint32_t tile = blockIdx.x;; tile += gridDim.x) {
+    uint32_t k, row, least;
+    Q.locate(tile, k, row, least);
+    if ((uint64_t)least * blockDim.x >= longest) break;
+    const uint32_t off = row * blockDim.x, n_k = Q.size(k);
+    if (off >= n_k) continue;  // this segment is shorter
+    const uint32_t k_out = Q.shift ? k : (tile >> kShardShift) & (kShards - 1u);
+    const bool live = off + threadIdx.x < n_k;
+    const uint32_t i = k * Q.cap + off + threadIdx.x;
     bool emit_next = false;
     float4 o_next, d_next, tp_next;
     bool tex_has = false;  // texel gradient of this lane's lookup, scattered below by the whole wave
     uint32_t tex_gi[4] = {0u, 0u, 0u, 0u};
     float *tex_a[4] = {nullptr, nullptr, nullptr, nullptr};
     float tex_w[4] = {0.f, 0.f, 0.f, 0.f}, tex_g[3] = {0.f, 0.f, 0.f};
-    if (i < count) {
+    if (live) {
       const float4 ro = ray_o[i], rd = ray_d[i];
       const float4 tpv = b == 0 ? make_float4(1.f, 1.f, 1.f, 0.f) : tp_in[i];  // a new path's throughput
       const uint32_t n = fbits(ro.w), slot = fbits(rd.w);
@@ -1785,7 +1881,7 @@ __global__ __launch_bounds__(256) void k_shade_adjoint(int32_t b, const uint32_t
     }
     if (kTex) scatter_texel_grads(tex_has, tex_a, tex_gi, tex_w, tex_g);
     uint32_t qn, unused;
-    block_append2(emit_next, next_count, false, next_count, qn, unused);
+    block_append2(emit_next, false, k_out, pairs, cap, qn, unused);
     if (emit_next) {
       nro[qn] = o_next;
       nrd[qn] = d_next;
@@ -2457,15 +2553,24 @@ struct TraceScratch {
   int max_grid = 0;  // 0: no cap beyond the persistent grid
 };
 
+QueueIn queue_of(uint32_t n) { return QueueIn{nullptr, n, 0u, 0u}; }
+// The rays of bounce b of a pass, and the shadow rays of its shading, by the
+// pass's counters; cap: the segments' entries.
+QueueIn ray_queue(const uint32_t *counts, int32_t b, uint32_t cap) {
+  return b == 0 ? QueueIn{counts, 0u, 0u, 0u} : QueueIn{counts + pair_word(b - 1), 0u, kShardShift, cap};
+}
+QueueIn shadow_queue(const uint32_t *counts, int32_t b, uint32_t cap) {
+  return QueueIn{counts + pair_word(b) + 1, 0u, kShardShift, cap};
+}
+
 template <bool kHasTmax, bool kInst, int kLds, bool kCount = false, bool kLdsScene = false>
-void launch_closest_t(gi_ctx *ctx, int grid, int block, const uint32_t *count_ptr, uint32_t count_host,
-                      const float4 *ro, const float4 *rd, float4 *hits, const TraceScratch &ts) {
+void launch_closest_t(gi_ctx *ctx, int grid, int block, const QueueIn &Q, const float4 *ro, const float4 *rd, float4 *hits, const TraceScratch &ts) {
   constexpr int kRows = stack_rows(kLds, kLdsScene, true);
   const size_t stack_bytes = trace_lds_bytes(kRows, block, !kLdsScene);
   const size_t scene_bytes =
       kLdsScene ? (size_t)ctx->nnodes * sizeof(WideNode) + (size_t)ctx->ntri * sizeof(IsectTri) : 0;
   hipLaunchKernelGGL((k_trace_closest<kHasTmax, kInst, kRows, kCount, kLdsScene>), dim3(grid), dim3(block),
-                     stack_bytes + scene_bytes, ctx->stream, count_ptr, count_host, ro, rd, hits,
+                     stack_bytes + scene_bytes, ctx->stream, Q, ro, rd, hits,
                      ctx->d_hnodes.as<HalfNode>(), ctx->d_nodes.as<WideNode>(), ctx->d_itris.as<float4>(),
                      ts.gstack ? ts.gstack : ctx->d_gstack.as<uint32_t>(), ctx->stack_cap,
                      ts.overflow ? ts.overflow : ctx->d_overflow.as<uint32_t>(), inst_scene(ctx),
@@ -2474,15 +2579,14 @@ void launch_closest_t(gi_ctx *ctx, int grid, int block, const uint32_t *count_pt
 }
 
 template <bool kDeposit, bool kInst, int kLds, bool kCount = false, bool kLdsScene = false>
-void launch_any_t(gi_ctx *ctx, int grid, int block, const uint32_t *count_ptr, uint32_t count_host,
-                  const float4 *ro, const float4 *rd, const float4 *contrib, float4 *pl, uint8_t *occ, float4 *rec,
+void launch_any_t(gi_ctx *ctx, int grid, int block, const QueueIn &Q, const float4 *ro, const float4 *rd, const float4 *contrib, float4 *pl, uint8_t *occ, float4 *rec,
                   uint32_t rec_stride, int32_t b) {
   constexpr int kRows = stack_rows(kLds, kLdsScene, false);
   const size_t stack_bytes = trace_lds_bytes(kRows, block, false);
   const size_t scene_bytes =
       kLdsScene ? (size_t)ctx->nnodes * sizeof(WideNode) + (size_t)ctx->ntri * sizeof(IsectTri) : 0;
   hipLaunchKernelGGL((k_trace_any<kDeposit, kInst, kRows, kCount, kLdsScene>), dim3(grid), dim3(block),
-                     stack_bytes + scene_bytes, ctx->stream, count_ptr, count_host, ro, rd, contrib, pl, occ,
+                     stack_bytes + scene_bytes, ctx->stream, Q, ro, rd, contrib, pl, occ,
                      ctx->d_hnodes.as<HalfNode>(), ctx->d_nodes.as<WideNode>(), ctx->d_itris.as<float4>(),
                      ctx->d_gstack.as<uint32_t>(),
                      ctx->stack_cap, ctx->d_overflow.as<uint32_t>(), rec, rec_stride, b, inst_scene(ctx),
@@ -2497,7 +2601,7 @@ int stack_lds_of(const gi_ctx *ctx) {
 
 bool instanced(const gi_ctx *ctx);
 
-int launch_closest(gi_ctx *ctx, bool has_tmax, const uint32_t *count_ptr, uint32_t count_host, uint64_t n_bound,
+int launch_closest(gi_ctx *ctx, bool has_tmax, const QueueIn &Q, uint64_t n_bound,
                    const float4 *ro, const float4 *rd, float4 *hits, const TraceScratch &ts = TraceScratch{}) {
   int grid, block;
   int rc = trace_grid_for(ctx, n_bound, grid, block);
@@ -2505,12 +2609,12 @@ int launch_closest(gi_ctx *ctx, bool has_tmax, const uint32_t *count_ptr, uint32
   if (ts.max_grid > 0) grid = std::min(grid, ts.max_grid);
   const int L = stack_lds_of(ctx);
   const bool I = instanced(ctx);
-#define GI_CL(T, II, LL) launch_closest_t<T, II, LL>(ctx, grid, block, count_ptr, count_host, ro, rd, hits, ts)
+#define GI_CL(T, II, LL) launch_closest_t<T, II, LL>(ctx, grid, block, Q, ro, rd, hits, ts)
 #define GI_CL_L(T, II) \
   if (ctx->count_traversal) \
-    launch_closest_t<T, II, 16, true>(ctx, grid, block, count_ptr, count_host, ro, rd, hits, ts); \
+    launch_closest_t<T, II, 16, true>(ctx, grid, block, Q, ro, rd, hits, ts); \
   else if (!(II) && L == 16 && lds_scene_of(ctx)) \
-    launch_closest_t<T, false, 16, false, true>(ctx, grid, block, count_ptr, count_host, ro, rd, hits, ts); \
+    launch_closest_t<T, false, 16, false, true>(ctx, grid, block, Q, ro, rd, hits, ts); \
   else if (L == 8) GI_CL(T, II, 8); \
   else if (L == 32) GI_CL(T, II, 32); \
   else GI_CL(T, II, 16)
@@ -2525,7 +2629,7 @@ int launch_closest(gi_ctx *ctx, bool has_tmax, const uint32_t *count_ptr, uint32
   return GI_OK;
 }
 
-int launch_any(gi_ctx *ctx, bool deposit, const uint32_t *count_ptr, uint32_t count_host, uint64_t n_bound,
+int launch_any(gi_ctx *ctx, bool deposit, const QueueIn &Q, uint64_t n_bound,
                const float4 *ro, const float4 *rd, const float4 *contrib, float4 *pl, uint8_t *occ,
                float4 *rec = nullptr, uint32_t rec_stride = 0, int32_t b = 0) {
   int grid, block;
@@ -2534,13 +2638,13 @@ int launch_any(gi_ctx *ctx, bool deposit, const uint32_t *count_ptr, uint32_t co
   const int L = stack_lds_of(ctx);
   const bool I = instanced(ctx);
 #define GI_ANY(D, II, LL) \
-  launch_any_t<D, II, LL>(ctx, grid, block, count_ptr, count_host, ro, rd, contrib, pl, occ, rec, rec_stride, b)
+  launch_any_t<D, II, LL>(ctx, grid, block, Q, ro, rd, contrib, pl, occ, rec, rec_stride, b)
 #define GI_ANY_L(D, II) \
   if (ctx->count_traversal) \
-    launch_any_t<D, II, 16, true>(ctx, grid, block, count_ptr, count_host, ro, rd, contrib, pl, occ, rec, rec_stride, \
+    launch_any_t<D, II, 16, true>(ctx, grid, block, Q, ro, rd, contrib, pl, occ, rec, rec_stride, \
                                   b); \
   else if (!(II) && L == 16 && lds_scene_of(ctx)) \
-    launch_any_t<D, false, 16, false, true>(ctx, grid, block, count_ptr, count_host, ro, rd, contrib, pl, occ, rec, \
+    launch_any_t<D, false, 16, false, true>(ctx, grid, block, Q, ro, rd, contrib, pl, occ, rec, \
                                             rec_stride, b); \
   else if (L == 8) GI_ANY(D, II, 8); \
   else if (L == 32) GI_ANY(D, II, 32); \
@@ -2628,8 +2732,11 @@ int ensure_workspace(gi_ctx *ctx, size_t slots) {
     if (ctx->textured) GI_HIP(ctx, ctx->rdiff.ensure(4 * ctx->slot_cap * sizeof(float4)));
     return GI_OK;
   }
-  const size_t b4 = slots * sizeof(float4);
-  if (ctx->textured) GI_HIP(ctx, ctx->rdiff.ensure(4 * b4));
+  // path state by slot; kShards segments of segment_cap entries are at most
+  // kShards tiles each longer, whatever the tile (at most 256)
+  const size_t p4 = slots * sizeof(float4);
+  const size_t b4 = (slots + (size_t)kShards * kShards * 256) * sizeof(float4);
+  if (ctx->textured) GI_HIP(ctx, ctx->rdiff.ensure(4 * p4));
   for (int i = 0; i < 2; ++i) {
     GI_HIP(ctx, ctx->q_o[i].ensure(b4));
     GI_HIP(ctx, ctx->q_d[i].ensure(b4));
@@ -2639,7 +2746,7 @@ int ensure_workspace(gi_ctx *ctx, size_t slots) {
   GI_HIP(ctx, ctx->s_o.ensure(b4));
   GI_HIP(ctx, ctx->s_d.ensure(b4));
   GI_HIP(ctx, ctx->s_c.ensure(b4));
-  GI_HIP(ctx, ctx->path_l.ensure(b4));
+  GI_HIP(ctx, ctx->path_l.ensure(p4));
   ctx->slot_cap = slots;
   return GI_OK;
 }
@@ -2744,6 +2851,22 @@ void drop_graph(gi_ctx *ctx) {
   ctx->graph_key.clear();
 }
 
+// Sum of word w (0: rays, 1: shadow rays) of a bounce's counter pairs.
+uint32_t sum_counts(const uint32_t *pairs, int w) {
+  uint32_t n = 0;
+  for (uint32_t k = 0; k < kShards; ++k) n += pairs[k * kCountStride + w];
+  return n;
+}
+// The rays of a pass by its counters: the slots and the rays its bounces
+// appended (those of the last bounce are none), and the shadow rays.
+void add_ray_counts(gi_ctx *ctx, const uint32_t *counts, int32_t depth) {
+  ctx->counters.rays_closest += counts[0];
+  for (int32_t b = 0; b < depth; ++b) {
+    ctx->counters.rays_closest += sum_counts(counts + pair_word(b), 0);
+    ctx->counters.rays_shadow += sum_counts(counts + pair_word(b), 1);
+  }
+}
+
 // The launches of the passes on the context stream.  sync_counts: read
 // every bounce's queue length back to the host and size the launches
 // exactly (the reference's synchronous, per-view flow); otherwise every
@@ -2753,7 +2876,7 @@ void drop_graph(gi_ctx *ctx) {
 template <class Mark>
 int enqueue_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, bool sync_counts, const ShadeParams &SP,
                    int &launches, Mark mark) {
-  const int32_t ncnt = 2 * depth + 1;  // ray queue counts [0..depth], shadow counts
+  const int32_t ncnt = count_words(depth);
   const size_t npass = plan.passes.size();
   const PassDesc *dpass = ctx->d_passes.as<PassDesc>();
   const DevView *dviews = ctx->d_views.as<DevView>();
@@ -2771,41 +2894,42 @@ int enqueue_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, bool sync_c
     hipLaunchKernelGGL(k_raygen, dim3(std::max(1, rg)), dim3(256), 0, ctx->stream, dp, dviews, SP.H,
                        ctx->q_o[0].as<float4>(), ctx->q_d[0].as<float4>(), ctx->path_l.as<float4>(),
                        (float4 *)nullptr, 0u, depth);
+    const uint32_t cap = segment_cap(pd.total_slots, (uint32_t)sblock);
     uint32_t host_count = pd.total_slots;
     for (int32_t b = 0; b < depth; ++b) {
       const int cur = b & 1, nxt = cur ^ 1;
-      if (sync_counts && b > 0) {
-        GI_HIP(ctx, hipMemcpyAsync(&host_count, cnt + b, 4, hipMemcpyDeviceToHost, ctx->stream));
-        GI_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (host_count == 0) break;
-      }
+      if (sync_counts && host_count == 0) break;
       const uint64_t bound = sync_counts ? host_count : pd.total_slots;
       if ((rc = mark(-1))) return rc;
-      rc = launch_closest(ctx, false, cnt + b, 0, bound, ctx->q_o[cur].as<float4>(),
+      rc = launch_closest(ctx, false, ray_queue(cnt, b, cap), bound, ctx->q_o[cur].as<float4>(),
                           ctx->q_d[cur].as<float4>(), ctx->q_hit.as<float4>());
       if (rc) return rc;
       ++launches;
       if ((rc = mark(0))) return rc;
-      const int sg = (int)std::max<uint64_t>(1, std::min<uint64_t>((bound + sblock - 1) / sblock, (uint64_t)persist));
+      // eight times the blocks the chip holds at once: they start out of
+      // step, and the last wave is short
+      const int sg = (int)std::max<uint64_t>(
+          1, std::min<uint64_t>((bound + sblock - 1) / sblock, (uint64_t)ctx->num_cus * 64));
       const bool phong = (ctx->opts.flags & GI_FLAG_PHONG) != 0;
       hipLaunchKernelGGL(phong ? (SP.rdiff ? k_shade_phong_tex : k_shade_phong) : (SP.rdiff ? k_shade_tex : k_shade),
                          dim3(sg), dim3(sblock), 0, ctx->stream, b,
-                         cnt + b, SPp, ctx->q_o[cur].as<float4>(), ctx->q_d[cur].as<float4>(),
+                         ray_queue(cnt, b, cap), SPp, ctx->q_o[cur].as<float4>(), ctx->q_d[cur].as<float4>(),
                          ctx->q_tp[cur].as<float4>(), ctx->q_hit.as<float4>(), ctx->path_l.as<float4>(),
                          ctx->q_o[nxt].as<float4>(), ctx->q_d[nxt].as<float4>(), ctx->q_tp[nxt].as<float4>(),
-                         cnt + b + 1, ctx->s_o.as<float4>(), ctx->s_d.as<float4>(), ctx->s_c.as<float4>(),
-                         cnt + depth + 1 + b, (float4 *)nullptr, 0u);
+                         cnt + pair_word(b), cap, ctx->s_o.as<float4>(), ctx->s_d.as<float4>(),
+                         ctx->s_c.as<float4>(), (float4 *)nullptr, 0u);
       GI_HIP(ctx, hipGetLastError());
       if ((rc = mark(2))) return rc;
-      uint32_t shadow_host = 0;
       uint64_t sbound = bound;
       if (sync_counts) {
-        GI_HIP(ctx, hipMemcpyAsync(&shadow_host, cnt + depth + 1 + b, 4, hipMemcpyDeviceToHost, ctx->stream));
+        uint32_t pairs[kShards * kCountStride];
+        GI_HIP(ctx, hipMemcpyAsync(pairs, cnt + pair_word(b), sizeof(pairs), hipMemcpyDeviceToHost, ctx->stream));
         GI_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        sbound = shadow_host;
+        host_count = sum_counts(pairs, 0);
+        sbound = sum_counts(pairs, 1);
       }
       if (sbound > 0) {
-        rc = launch_any(ctx, true, cnt + depth + 1 + b, 0, sbound, ctx->s_o.as<float4>(), ctx->s_d.as<float4>(),
+        rc = launch_any(ctx, true, shadow_queue(cnt, b, cap), sbound, ctx->s_o.as<float4>(), ctx->s_d.as<float4>(),
                         ctx->s_c.as<float4>(), ctx->path_l.as<float4>(), nullptr);
         if (rc) return rc;
       }
@@ -2824,7 +2948,7 @@ int enqueue_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, bool sync_c
 // whose launches take the same arguments (launch_key); otherwise it is
 // captured and instantiated again (counters.ms_graph_build).
 int run_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, bool sync_counts, bool use_graph, bool timing) {
-  const int32_t ncnt = 2 * depth + 1;
+  const int32_t ncnt = count_words(depth);
   const size_t npass = plan.passes.size();
   GI_HIP(ctx, ctx->d_passes.ensure(npass * sizeof(PassDesc)));
   GI_HIP(ctx, hipMemcpyAsync(ctx->d_passes.p, plan.passes.data(), npass * sizeof(PassDesc), hipMemcpyHostToDevice,
@@ -2895,12 +3019,7 @@ int run_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, bool sync_count
   // telemetry
   std::vector<uint32_t> hc(npass * ncnt);
   GI_HIP(ctx, copy_sync(ctx, hc.data(), ctx->d_counters.p, hc.size() * 4, hipMemcpyDeviceToHost));
-  for (size_t pi = 0; pi < npass; ++pi) {
-    for (int32_t b = 0; b < depth; ++b) {
-      ctx->counters.rays_closest += hc[pi * ncnt + b];
-      ctx->counters.rays_shadow += hc[pi * ncnt + depth + 1 + b];
-    }
-  }
+  for (size_t pi = 0; pi < npass; ++pi) add_ray_counts(ctx, hc.data() + pi * ncnt, depth);
   ctx->counters.ms_trace_closest += ms_c;
   ctx->counters.ms_trace_any += ms_a;
   ctx->counters.ms_shade += ms_s;
@@ -2915,7 +3034,7 @@ int run_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, bool sync_count
 // that accumulates the gradients.  Device-side queue lengths, persistent
 // grids, no host synchronisation until the end.
 int run_adjoint_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, AdjParams A) {
-  const int32_t ncnt = 2 * depth + 1;
+  const int32_t ncnt = count_words(depth);
   const size_t npass = plan.passes.size();
   GI_HIP(ctx, ctx->d_passes.ensure(npass * sizeof(PassDesc)));
   GI_HIP(ctx, hipMemcpyAsync(ctx->d_passes.p, plan.passes.data(), npass * sizeof(PassDesc), hipMemcpyHostToDevice,
@@ -2943,6 +3062,7 @@ int run_adjoint_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, AdjPara
     const PassDesc &pd = plan.passes[pi];
     const PassDesc *dp = dpass + pi;
     A.pass = dp;
+    const uint32_t cap = segment_cap(pd.total_slots, (uint32_t)sblock);
     ShadeParams SPp = SP;
     SPp.pass = dp;
     const int rg = (int)std::min<uint64_t>((pd.total_slots + 255) / 256, (uint64_t)persist);
@@ -2958,27 +3078,27 @@ int run_adjoint_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, AdjPara
         const int cur = b & 1, nxt = cur ^ 1;
         if (phase == 0) {
           // the replay (phase 1) reads these hits from the record
-          rc = launch_closest(ctx, false, cnt + b, 0, pd.total_slots, ctx->q_o[cur].as<float4>(),
+          rc = launch_closest(ctx, false, ray_queue(cnt, b, cap), pd.total_slots, ctx->q_o[cur].as<float4>(),
                               ctx->q_d[cur].as<float4>(), ctx->q_hit.as<float4>());
           if (rc) return rc;
           hipLaunchKernelGGL(SP.rdiff ? k_shade_tex : k_shade, dim3(sg), dim3(sblock), 0, ctx->stream, b,
-                             cnt + b, SPp,
+                             ray_queue(cnt, b, cap), SPp,
                              ctx->q_o[cur].as<float4>(), ctx->q_d[cur].as<float4>(), ctx->q_tp[cur].as<float4>(),
                              ctx->q_hit.as<float4>(), ctx->path_l.as<float4>(), ctx->q_o[nxt].as<float4>(),
-                             ctx->q_d[nxt].as<float4>(), ctx->q_tp[nxt].as<float4>(), cnt + b + 1,
+                             ctx->q_d[nxt].as<float4>(), ctx->q_tp[nxt].as<float4>(), cnt + pair_word(b), cap,
                              ctx->s_o.as<float4>(), ctx->s_d.as<float4>(), ctx->s_c.as<float4>(),
-                             cnt + depth + 1 + b, rec, stride);
+                             rec, stride);
           GI_HIP(ctx, hipGetLastError());
-          rc = launch_any(ctx, true, cnt + depth + 1 + b, 0, pd.total_slots, ctx->s_o.as<float4>(),
+          rc = launch_any(ctx, true, shadow_queue(cnt, b, cap), pd.total_slots, ctx->s_o.as<float4>(),
                           ctx->s_d.as<float4>(), ctx->s_c.as<float4>(), ctx->path_l.as<float4>(), nullptr, rec,
                           stride, b);
           if (rc) return rc;
         } else {
           hipLaunchKernelGGL(SP.rdiff ? k_shade_adjoint<true> : k_shade_adjoint<false>, dim3(sg), dim3(sblock),
-                             lds_adj, ctx->stream, b, cnt + b, SPp, A,
+                             lds_adj, ctx->stream, b, ray_queue(cnt, b, cap), SPp, A,
                              ctx->q_o[cur].as<float4>(), ctx->q_d[cur].as<float4>(), ctx->q_tp[cur].as<float4>(),
                              ctx->q_o[nxt].as<float4>(), ctx->q_d[nxt].as<float4>(),
-                             ctx->q_tp[nxt].as<float4>(), cnt + b + 1);
+                             ctx->q_tp[nxt].as<float4>(), cnt + pair_word(b), cap);
           GI_HIP(ctx, hipGetLastError());
         }
       }
@@ -2988,10 +3108,7 @@ int run_adjoint_passes(gi_ctx *ctx, const PassPlan &plan, int32_t depth, AdjPara
   std::vector<uint32_t> hc(2 * npass * ncnt);
   GI_HIP(ctx, copy_sync(ctx, hc.data(), ctx->d_counters.p, hc.size() * 4, hipMemcpyDeviceToHost));
   for (size_t k = 0; k < 2 * npass; k += 2)  // the forward (recording) phases trace; the replays do not
-    for (int32_t b = 0; b < depth; ++b) {
-      ctx->counters.rays_closest += hc[k * ncnt + b];
-      ctx->counters.rays_shadow += hc[k * ncnt + depth + 1 + b];
-    }
+    add_ray_counts(ctx, hc.data() + k * ncnt, depth);
   ctx->counters.passes += (int32_t)npass;
   return check_overflow(ctx);
 }
@@ -3731,7 +3848,7 @@ int gi_trace_closest_device(gi_ctx *ctx, const float *d_orig, const float *d_dir
   hipLaunchKernelGGL(k_pack_rays, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, ctx->stream, d_orig, d_dir,
                      d_max_t, (uint32_t)n, ctx->p_ro.as<float4>(), ctx->p_rd.as<float4>());
   GI_HIP(ctx, hipGetLastError());
-  rc = launch_closest(ctx, true, nullptr, (uint32_t)n, (uint64_t)n, ctx->p_ro.as<float4>(), ctx->p_rd.as<float4>(),
+  rc = launch_closest(ctx, true, queue_of((uint32_t)n), (uint64_t)n, ctx->p_ro.as<float4>(), ctx->p_rd.as<float4>(),
                       reinterpret_cast<float4 *>(d_out));
   if (rc) return rc;
   GI_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -3755,7 +3872,7 @@ int gi_trace_any_device(gi_ctx *ctx, const float *d_orig, const float *d_dir, co
   hipLaunchKernelGGL(k_pack_rays, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, ctx->stream, d_orig, d_dir,
                      d_max_t, (uint32_t)n, ctx->p_ro.as<float4>(), ctx->p_rd.as<float4>());
   GI_HIP(ctx, hipGetLastError());
-  rc = launch_any(ctx, false, nullptr, (uint32_t)n, (uint64_t)n, ctx->p_ro.as<float4>(), ctx->p_rd.as<float4>(),
+  rc = launch_any(ctx, false, queue_of((uint32_t)n), (uint64_t)n, ctx->p_ro.as<float4>(), ctx->p_rd.as<float4>(),
                   nullptr, nullptr, d_occluded);
   if (rc) return rc;
   GI_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -3792,7 +3909,7 @@ int gi_trace_closest_device_noalloc(gi_ctx *ctx, const float *d_orig, const floa
   hipLaunchKernelGGL(k_pack_rays, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, ctx->stream, d_orig, d_dir,
                      d_max_t, (uint32_t)n, ro, rd);
   GI_HIP(ctx, hipGetLastError());
-  rc = launch_closest(ctx, true, nullptr, (uint32_t)n, (uint64_t)n, ro, rd, reinterpret_cast<float4 *>(d_out), ts);
+  rc = launch_closest(ctx, true, queue_of((uint32_t)n), (uint64_t)n, ro, rd, reinterpret_cast<float4 *>(d_out), ts);
   if (rc) return rc;
   uint32_t ov = 0;
   GI_HIP(ctx, hipMemcpyAsync(&ov, overflow, 4, hipMemcpyDeviceToHost, ctx->stream));

@@ -127,3 +127,23 @@ def test_lds_scene_matches_global_path(oracle, gpu_ctx_factory):
         bad = np.nonzero(out[16][1] != ref_hits)[0]
         assert len(bad) <= 2  # FP64 ties only, as in the other parity tests
         assert np.array_equal(out[16][2].astype(bool), ref_occ.astype(bool))
+
+
+@pytest.mark.parametrize("shade_block", [64, 128, 192, 256])
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (17, 15, 1), (257, 1, 1), (17, 241, 1), (129, 127, 3)])
+def test_queue_segments(w, h, spp, shade_block, oracle, gpu_ctx_factory):
+    """Path counts around the edges of shading tiles and of the queues'
+    segment groups, for every tile size: images and ray counts are the
+    oracle's with the counts read back per bounce, on the device and in a
+    replayed graph."""
+    sc = scenes.cornell_boxes(w=w, h=h, spp=spp, depth=6)
+    sc.opts["rr_start"] = 2
+    ref, st = oracle.OracleScene(sc.tris, sc.mats, sc.lights).render(sc.views, sc.opts)
+    with gpu_ctx_factory() as ctx:
+        ctx.set_tuning(shade_block=shade_block)
+        ctx.upload(sc)
+        for flags in (0, FLAG_BATCHED, FLAG_BATCHED | FLAG_GRAPH, FLAG_BATCHED | FLAG_GRAPH):
+            img = ctx.render(flags=flags).image(0).reshape(-1, 3)
+            c = ctx.counters()
+            assert (img == ref).all(), flags
+            assert (c["rays_closest"], c["rays_shadow"]) == (st["rays_closest"], st["rays_shadow"]), flags
