@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from globillum_amd import autotune, scenes
-from globillum_amd._lib import FLAG_BATCHED, GiError
+from globillum_amd._lib import FLAG_BATCHED, FLAG_GRAPH, GiError
 
 pytestmark = pytest.mark.gpu
 FMAX = np.finfo(np.float32).max
