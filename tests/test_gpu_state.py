@@ -233,3 +233,18 @@ def test_trace_device_entry_points_on_device_buffers(oracle, gpu_ctx_factory):
     from test_gpu_trace import _assert_hits_equal
     _assert_hits_equal(got, ref, osc, o, d, t)
     assert np.array_equal(got_any, ref_any)
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (5, 3), (255, 1), (257, 255), (256, 256), (65537, 1), (1024, 512),
+                                 (1023, 1025), (4099, 131)])
+def test_image_readback_sizes(w, h, oracle, gpu_ctx_factory):
+    """gi_get_image around the sizes of its blocks, chunks (65536 pixels) and
+    slots (8 chunks): every pixel of the oracle's image, bit for bit, also
+    into a caller's buffer that is only 4-byte aligned."""
+    sc = scenes.cornell_boxes(w=w, h=h, spp=1, depth=1)
+    ref, _ = oracle.OracleScene(sc.tris, sc.mats, sc.lights).render(sc.views, sc.opts)
+    with gpu_ctx_factory(sc) as ctx:
+        assert (ctx.render().image(0).reshape(-1, 3) == ref).all()
+        out = np.zeros(3 * w * h + 1, np.float32)
+        assert ctx.lib.gi_get_image(ctx.h, 0, ptr(out[1:])) == 0
+        assert (out[1:].reshape(-1, 3) == ref).all() and out[0] == 0
