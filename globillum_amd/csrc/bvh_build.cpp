@@ -84,6 +84,16 @@ struct Builder {
       for (int k = 0; k < 3; ++k) cen[3 * i + k] = 0.5f * (tbox[i].lo[k] + tbox[i].hi[k]);
     }
   }
+  // over the boxes of triangles, as the first constructor makes them
+  Builder(const TriBox *t, int64_t n, int32_t ml, std::vector<uint32_t> &p, std::vector<Bvh2Node> &nd)
+      : tris(nullptr), tbox(n), cen(3 * n), perm(p), nodes(nd), max_leaf(ml) {
+    for (int64_t i = 0; i < n; ++i)
+      for (int k = 0; k < 3; ++k) {
+        tbox[i].lo[k] = t[i].lo[k];
+        tbox[i].hi[k] = t[i].hi[k];
+        cen[3 * i + k] = 0.5f * (tbox[i].lo[k] + tbox[i].hi[k]);
+      }
+  }
   // over arbitrary boxes (lo xyz, hi xyz per primitive)
   Builder(const float *boxes, int64_t n, int32_t ml, std::vector<uint32_t> &p, std::vector<Bvh2Node> &nd)
       : tris(nullptr), tbox(n), cen(3 * n), perm(p), nodes(nd), max_leaf(ml) {
@@ -237,7 +247,9 @@ inline float bitsf(int32_t i) {
 
 }  // namespace
 
-void build_bvh2(const gi_tri *tris, int64_t n, int32_t max_leaf, gi_bvh &out, int32_t threads) {
+namespace {
+// The binned-SAH build over triangles, or over their boxes.
+template <class Prim> void build_sah(const Prim *prims, int64_t n, int32_t max_leaf, gi_bvh &out, int32_t threads) {
   out.nodes.clear();
   out.perm.resize(n);
   std::iota(out.perm.begin(), out.perm.end(), 0u);
@@ -249,10 +261,19 @@ void build_bvh2(const gi_tri *tris, int64_t n, int32_t max_leaf, gi_bvh &out, in
     out.max_depth = 0;
     return;
   }
-  Builder bld(tris, n, max_leaf, out.perm, out.nodes);
+  Builder bld(prims, n, max_leaf, out.perm, out.nodes);
   bld.parallel = threads != 1;
   bld.build(0, 0, (uint32_t)n, 0);
   out.max_depth = bld.max_depth;
+}
+}  // namespace
+
+void build_bvh2(const gi_tri *tris, int64_t n, int32_t max_leaf, gi_bvh &out, int32_t threads) {
+  build_sah(tris, n, max_leaf, out, threads);
+}
+
+void build_bvh2(const TriBox *boxes, int64_t n, int32_t max_leaf, gi_bvh &out, int32_t threads) {
+  build_sah(boxes, n, max_leaf, out, threads);
 }
 
 void build_bvh2_boxes(const float *boxes, int64_t n, int32_t max_leaf, gi_bvh &out, int32_t threads) {

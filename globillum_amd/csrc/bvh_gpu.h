@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <string>
 
 #include "gi_internal.h"
@@ -25,7 +26,9 @@ enum class DeviceBvhMethod { kLbvh = 0, kPloc = 1, kSah = 2 };
 // radix tree over the Morton keys; kPloc: clustering with the given search
 // radius (1..64); kSah: the host builder's binned SAH (clo, chi and radius
 // unused).  width: child slots filled per wide node (2..4).  Synchronises
-// the stream; scratch memory is allocated and freed inside.
+// the stream.  Its scratch memory is one block that `scratch` returns for a
+// size (null: out of memory), used until the return; a segmented sort's
+// buffers, which few trees need, are allocated and freed inside.
 // The 3n float4 of the leaf-ordered intersection triangles (a with the
 // original index in w, b - a, c - a) from the ShadeTri-strided vertex table
 // and a leaf-order permutation already on the device.  Asynchronous.
@@ -34,6 +37,7 @@ hipError_t launch_leaf_tris(hipStream_t s, const float4 *tri, uint32_t stride, u
 
 bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_t n, const float clo[3],
                       const float chi[3], int max_leaf, DeviceBvhMethod method, int radius, int width,
-                      WideNode *nodes, float4 *itris, LbvhResult &res, std::string &err);
+                      WideNode *nodes, float4 *itris, const std::function<void *(size_t)> &scratch, LbvhResult &res,
+                      std::string &err);
 
 }  // namespace gi

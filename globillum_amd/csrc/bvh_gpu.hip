@@ -1256,6 +1256,24 @@ __global__ void k_sah_last(uint32_t *__restrict__ ne, uint32_t nodes) {
     }                                                                 \
   } while (0)
 
+// Places arrays one after another (256-byte aligned) in one block: carved
+// once without a block for its size, then again in the block.
+struct Carver {
+  uint8_t *base = nullptr;
+  size_t used = 0;
+  void *bytes(size_t n) {
+    void *p = base ? base + used : nullptr;
+    used += (std::max<size_t>(n, 16) + 255) & ~(size_t)255;
+    return p;
+  }
+  template <class T> void get(T *&p, size_t n) { p = static_cast<T *>(bytes(n * sizeof(T))); }
+  bool take(const std::function<void *(size_t)> &scratch) {
+    base = static_cast<uint8_t *>(scratch(used));
+    used = 0;
+    return base != nullptr;
+  }
+};
+
 hipError_t launch_leaf_tris(hipStream_t s, const float4 *tri, uint32_t stride, uint32_t n, const uint32_t *order,
                             float4 *itris) {
   if (n == 0) return hipSuccess;
@@ -1329,7 +1347,8 @@ static bool emit_wide(hipStream_t s, const CollapseArgs &A, int32_t root, WideNo
 
 // The binned-SAH tree, level by level (kernels above), then the collapse.
 static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_t n, int max_leaf, int W,
-                             WideNode *nodes, float4 *itris, LbvhResult &res, std::string &err) {
+                             WideNode *nodes, float4 *itris, const std::function<void *(size_t)> &scratch, LbvhResult &res,
+                             std::string &err) {
   std::vector<void *> mem;
   auto alloc = [&](size_t bytes) -> void * {
     void *p = nullptr;
@@ -1340,55 +1359,61 @@ static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, 
   const size_t nn = 2 * (size_t)n;  // binary nodes: at most 2n - 1
   // a level lists the children of split nodes (more than max_leaf triangles each)
   const size_t lcap = std::min<size_t>(n, 2 * ((size_t)n / (max_leaf + 1)) + 2);
-  SahArgs S;
-  for (int b = 0; b < 2; ++b) {
-    S.box[b] = (float4 *)alloc(32 * (size_t)n);
-    S.perm[b] = (uint32_t *)alloc(4 * (size_t)n);
-    S.pos[b] = (int32_t *)alloc(4 * (size_t)n);
-  }
-  S.left = (int32_t *)alloc(4 * nn);
-  S.right = (int32_t *)alloc(4 * nn);
-  S.nb = (uint32_t *)alloc(4 * nn);
-  S.ne = (uint32_t *)alloc(4 * nn);
-  S.bb = (float4 *)alloc(32 * nn);
-  S.cb = (float4 *)alloc(32 * nn);
-  S.nodebox = (float *)alloc(32 * nn);
-  S.dec = (SahDec *)alloc(sizeof(SahDec) * lcap);
-  S.leaf_perm = (uint32_t *)alloc(4 * (size_t)n);
-  S.max_leaf = max_leaf;
-  int32_t *lvl = (int32_t *)alloc(4 * nn);  // every level's list, one after another
-  uint64_t *want = (uint64_t *)alloc(8 * lcap), *pre = (uint64_t *)alloc(8 * lcap);
-  uint32_t *flags = (uint32_t *)alloc(4 * (size_t)n), *scan = (uint32_t *)alloc(4 * (size_t)n);
   const size_t max_big = (size_t)n / kSahChunk + 1;  // nodes of several chunks per level
-  uint32_t *gbins = (uint32_t *)alloc(4 * (size_t)kSahBinWords * max_big);
-  uint32_t *big_pos = (uint32_t *)alloc(4 * max_big);
-  uint32_t *med_pos = (uint32_t *)alloc(4 * lcap), *seg_b = (uint32_t *)alloc(4 * lcap),
-           *seg_e = (uint32_t *)alloc(4 * lcap);
-  int32_t *med_kids = (int32_t *)alloc(8 * lcap);
-  float4 *cost = (float4 *)alloc(16 * nn);
-  uint32_t *meta = (uint32_t *)alloc(4 * nn);
-  int32_t *front[2] = {(int32_t *)alloc(4 * (size_t)n), (int32_t *)alloc(4 * (size_t)n)};
-  uint32_t *cnt = (uint32_t *)alloc(64);  // the collapse's counter; first the root's 12 box keys
-  uint32_t *tot = (uint32_t *)alloc(16);  // a level's chunk and several-chunk node counts
-  for (void *p : mem)
-    if (!p) {
-      err = "device bvh: out of device memory";
-      for (void *q : mem) (void)hipFree(q);
-      return false;
+  SahArgs S;
+  int32_t *lvl, *med_kids, *front[2];  // lvl: every level's list, one after another
+  uint64_t *want, *pre;
+  uint32_t *flags, *scan, *gbins, *big_pos, *med_pos, *seg_b, *seg_e, *meta, *cnt, *tot;
+  float4 *cost;
+  void *scan_temp;
+  size_t scan_bytes = 0, scan64_bytes = 0;
+  GI_CK(hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, (uint32_t *)nullptr, (uint32_t *)nullptr, (int)n, s));
+  GI_CK(hipcub::DeviceScan::ExclusiveSum(nullptr, scan64_bytes, (uint64_t *)nullptr, (uint64_t *)nullptr, (int)lcap, s));
+  Carver c;
+  const auto carve = [&] {
+    for (int b = 0; b < 2; ++b) {
+      c.get(S.box[b], 2 * (size_t)n);
+      c.get(S.perm[b], n);
+      c.get(S.pos[b], n);
+      c.get(front[b], n);
     }
+    c.get(S.left, nn);
+    c.get(S.right, nn);
+    c.get(S.nb, nn);
+    c.get(S.ne, nn);
+    c.get(S.bb, 2 * nn);
+    c.get(S.cb, 2 * nn);
+    c.get(S.nodebox, 8 * nn);
+    c.get(S.dec, lcap);
+    c.get(S.leaf_perm, n);
+    c.get(lvl, nn);
+    c.get(want, lcap);
+    c.get(pre, lcap);
+    c.get(flags, n);
+    c.get(scan, n);
+    c.get(gbins, (size_t)kSahBinWords * max_big);
+    c.get(big_pos, max_big);
+    c.get(med_pos, lcap);
+    c.get(seg_b, lcap);
+    c.get(seg_e, lcap);
+    c.get(med_kids, 2 * lcap);
+    c.get(cost, nn);
+    c.get(meta, nn);
+    c.get(cnt, 16);  // the collapse's counter; first the root's 12 box keys
+    c.get(tot, 4);   // a level's chunk and several-chunk node counts
+    scan_temp = c.bytes(std::max(scan_bytes, scan64_bytes));
+  };
+  carve();
+  if (!c.take(scratch)) {
+    err = "device bvh: out of device memory";
+    return false;
+  }
+  carve();
+  S.max_leaf = max_leaf;
   uint64_t *keys = nullptr, *keys2 = nullptr;  // median sort, allocated when a level needs it
   uint32_t *vals = nullptr, *vals2 = nullptr;
   void *sort_temp = nullptr;
   size_t sort_bytes = 0;
-  size_t scan_bytes = 0, scan64_bytes = 0;
-  GI_CK(hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, flags, scan, (int)n, s));
-  GI_CK(hipcub::DeviceScan::ExclusiveSum(nullptr, scan64_bytes, want, pre, (int)lcap, s));
-  void *scan_temp = alloc(std::max(scan_bytes, scan64_bytes));
-  if (!scan_temp) {
-    err = "device bvh: out of device memory (scan)";
-    for (void *q : mem) (void)hipFree(q);
-    return false;
-  }
   hipLaunchKernelGGL(k_sah_init, dim3(blocks(n)), dim3(kBlock), 0, s, tri, stride, n, S);
   const int32_t root = 0;
   const uint32_t range[2] = {0u, n};
@@ -1509,14 +1534,8 @@ static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, 
 
 bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_t n, const float clo[3],
                       const float chi[3], int max_leaf, DeviceBvhMethod method, int radius, int width, WideNode *nodes,
-                      float4 *itris, LbvhResult &res, std::string &err) {
-  std::vector<void *> mem;
-  auto alloc = [&](size_t bytes) -> void * {
-    void *p = nullptr;
-    if (hipMalloc(&p, std::max<size_t>(bytes, 16)) != hipSuccess) return nullptr;
-    mem.push_back(p);
-    return p;
-  };
+                      float4 *itris, const std::function<void *(size_t)> &scratch, LbvhResult &res, std::string &err) {
+  std::vector<void *> mem;  // none: the scratch block holds everything
   if (n == 0 || max_leaf < 1 || max_leaf > kMaxLeafTris) {
     err = "device bvh: n > 0 and 1 <= max_leaf <= 15 required";
     return false;
@@ -1526,49 +1545,75 @@ bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_
     return false;
   }
   if (method == DeviceBvhMethod::kSah)
-    return device_sah_build(s, tri, stride, n, max_leaf, std::max(2, std::min(4, width)), nodes, itris, res, err);
+    return device_sah_build(s, tri, stride, n, max_leaf, std::max(2, std::min(4, width)), nodes, itris, scratch,
+                            res, err);
   const bool ploc = method == DeviceBvhMethod::kPloc;
   const size_t ni = n > 1 ? n - 1 : 1;
-  // 30-bit keys for the radix tree, 63-bit keys for the clustering
-  uint32_t *keys = (uint32_t *)alloc(8 * (size_t)n), *keys2 = (uint32_t *)alloc(8 * (size_t)n);
-  uint32_t *vals = (uint32_t *)alloc(4 * (size_t)n), *vals2 = (uint32_t *)alloc(4 * (size_t)n);
-  int32_t *left = (int32_t *)alloc(4 * ni), *right = (int32_t *)alloc(4 * ni), *parent = (int32_t *)alloc(4 * ni);
-  int32_t *leaf_parent = (int32_t *)alloc(4 * (size_t)n);
-  uint32_t *first = (uint32_t *)alloc(4 * ni), *last = (uint32_t *)alloc(4 * ni);
-  int32_t *levels_buf = (int32_t *)alloc(4 * ni);  // radix tree nodes by breadth-first level
-  float *leafbox = (float *)alloc(32 * (size_t)n), *nodebox = (float *)alloc(32 * ni);
-  int32_t *front[2] = {(int32_t *)alloc(4 * ni), (int32_t *)alloc(4 * ni)};
-  uint32_t *cnt = (uint32_t *)alloc(16);
-  float4 *cost = (float4 *)alloc(16 * ni);  // the collapse's cost table and decisions
-  uint32_t *meta = (uint32_t *)alloc(4 * ni);
   const int W = std::max(2, std::min(4, width));
+  constexpr int kRoundsPerSync = 4;
+  // 30-bit keys for the radix tree, 63-bit keys for the clustering
+  uint32_t *keys, *keys2, *vals, *vals2, *first, *last, *cnt, *meta;
+  int32_t *left, *right, *parent, *leaf_parent, *levels_buf, *front[2];  // levels_buf: radix tree nodes by level
+  float *leafbox, *nodebox;
+  float4 *cost;  // the collapse's cost table and decisions (meta)
   // PLOC: clusters (double-buffered), their boxes, neighbours, round flags
   // and their scan, node leaf counts, leaf slots, the reordered leaves.
   int32_t *cl[2] = {nullptr, nullptr}, *nn = nullptr;
   float4 *cbox[2] = {nullptr, nullptr}, *leafbox2 = nullptr;
   uint64_t *flags = nullptr, *pre = nullptr;
   uint32_t *ncount = nullptr, *slot = nullptr, *order2 = nullptr, *round_log = nullptr;
-  constexpr int kRoundsPerSync = 4;
+  void *temp;
+  size_t temp_bytes = 0, scan_bytes = 0;
   if (ploc) {
-    round_log = (uint32_t *)alloc(4 * ((size_t)n + kRoundsPerSync + 1));  // rounds <= n - 1 + kRoundsPerSync
-    cl[0] = (int32_t *)alloc(4 * (size_t)n);
-    cl[1] = (int32_t *)alloc(4 * (size_t)n);
-    cbox[0] = (float4 *)alloc(32 * (size_t)n);
-    cbox[1] = (float4 *)alloc(32 * (size_t)n);
-    nn = (int32_t *)alloc(4 * (size_t)n);
-    flags = (uint64_t *)alloc(8 * (size_t)n);
-    pre = (uint64_t *)alloc(8 * (size_t)n);
-    ncount = (uint32_t *)alloc(4 * ni);
-    slot = (uint32_t *)alloc(4 * (size_t)n);
-    order2 = (uint32_t *)alloc(4 * (size_t)n);
-    leafbox2 = (float4 *)alloc(32 * (size_t)n);
+    GI_CK(hipcub::DeviceRadixSort::SortPairs(nullptr, temp_bytes, (uint64_t *)nullptr, (uint64_t *)nullptr,
+                                             (uint32_t *)nullptr, (uint32_t *)nullptr, (int)n, 0, 63, s));
+    GI_CK(hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, flags, pre, (int)n, s));
+  } else {
+    GI_CK(hipcub::DeviceRadixSort::SortPairs(nullptr, temp_bytes, (uint32_t *)nullptr, (uint32_t *)nullptr,
+                                             (uint32_t *)nullptr, (uint32_t *)nullptr, (int)n, 0, 30, s));
   }
-  for (void *p : mem)
-    if (!p) {
-      err = "device bvh: out of device memory";
-      for (void *q : mem) (void)hipFree(q);
-      return false;
+  Carver c;
+  const auto carve = [&] {
+    c.get(keys, 2 * (size_t)n);
+    c.get(keys2, 2 * (size_t)n);
+    c.get(vals, n);
+    c.get(vals2, n);
+    c.get(left, ni);
+    c.get(right, ni);
+    c.get(parent, ni);
+    c.get(leaf_parent, n);
+    c.get(first, ni);
+    c.get(last, ni);
+    c.get(levels_buf, ni);
+    c.get(leafbox, 8 * (size_t)n);
+    c.get(nodebox, 8 * ni);
+    c.get(front[0], ni);
+    c.get(front[1], ni);
+    c.get(cnt, 4);
+    c.get(cost, ni);
+    c.get(meta, ni);
+    if (ploc) {
+      c.get(round_log, (size_t)n + kRoundsPerSync + 1);  // rounds <= n - 1 + kRoundsPerSync
+      for (int b = 0; b < 2; ++b) {
+        c.get(cl[b], n);
+        c.get(cbox[b], 2 * (size_t)n);
+      }
+      c.get(nn, n);
+      c.get(flags, n);
+      c.get(pre, n);
+      c.get(ncount, ni);
+      c.get(slot, n);
+      c.get(order2, n);
+      c.get(leafbox2, 2 * (size_t)n);
     }
+    temp = c.bytes(std::max(temp_bytes, scan_bytes));
+  };
+  carve();
+  if (!c.take(scratch)) {
+    err = "device bvh: out of device memory";
+    return false;
+  }
+  carve();
   float3 lo = make_float3(clo[0], clo[1], clo[2]);
   float3 sc;
   sc.x = chi[0] > clo[0] ? 1.0f / (chi[0] - clo[0]) : 0.0f;
@@ -1578,17 +1623,6 @@ bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_
   if (ploc) hipLaunchKernelGGL(k_morton64, dim3(blocks(n)), dim3(kBlock), 0, s, tri, stride, n, lo, sc, keys64, vals);
   else hipLaunchKernelGGL(k_morton, dim3(blocks(n)), dim3(kBlock), 0, s, tri, stride, n, lo, sc, keys, vals);
   GI_CK(hipGetLastError());
-  size_t temp_bytes = 0, scan_bytes = 0;
-  if (ploc)
-    GI_CK(hipcub::DeviceRadixSort::SortPairs(nullptr, temp_bytes, keys64, keys64_2, vals, vals2, (int)n, 0, 63, s));
-  else GI_CK(hipcub::DeviceRadixSort::SortPairs(nullptr, temp_bytes, keys, keys2, vals, vals2, (int)n, 0, 30, s));
-  if (ploc) GI_CK(hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, flags, pre, (int)n, s));
-  void *temp = alloc(std::max(temp_bytes, scan_bytes));
-  if (!temp) {
-    err = "device bvh: out of device memory (sort)";
-    for (void *q : mem) (void)hipFree(q);
-    return false;
-  }
   if (ploc) GI_CK(hipcub::DeviceRadixSort::SortPairs(temp, temp_bytes, keys64, keys64_2, vals, vals2, (int)n, 0, 63, s));
   else GI_CK(hipcub::DeviceRadixSort::SortPairs(temp, temp_bytes, keys, keys2, vals, vals2, (int)n, 0, 30, s));
   const uint32_t *order = vals2;

@@ -91,6 +91,13 @@ namespace gi {
 // least 2^16 primitives near the root build on other threads.  Both give
 // the same nodes in the same order.
 void build_bvh2(const gi_tri *tris, int64_t n, int32_t max_leaf, gi_bvh &out, int32_t threads = 0);
+// The same build from the triangles' boxes: corner by corner, lo[k] =
+// min(lo[k], corner) from FLT_MAX and hi[k] = max(hi[k], corner) from
+// -FLT_MAX.
+struct TriBox {
+  float lo[3], hi[3];
+};
+void build_bvh2(const TriBox *boxes, int64_t n, int32_t max_leaf, gi_bvh &out, int32_t threads = 0);
 // Import a binary BVH in the reference's 2 x float4 layout.
 bool import_bvh2(const float *nodes, int64_t n_nodes, const uint32_t *indices, int64_t n_indices,
                  int64_t n_tris, gi_bvh &out, std::string &err);

@@ -21,6 +21,7 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -1954,6 +1955,104 @@ __global__ __launch_bounds__(256) void k_accumulate(const PassDesc *__restrict__
   }
 }
 
+// Triangle records (gi_tri, 25 floats) to the ShadeTri table, and per block
+// the bounds over its triangles: corners, centroids, material indices (14
+// words; the host folds the blocks').  A block stages 128 records in LDS
+// with coalesced 4-byte reads (the records are 100 bytes) and writes the
+// table as consecutive float4.  Minima and maxima are std::min / std::max in
+// operand order, so a NaN coordinate is passed over as the host's loop did.
+constexpr uint32_t kConvertTris = 128;
+struct TriBounds {
+  float lo[3], hi[3], clo[3], chi[3];
+  int32_t mat_lo, mat_hi;
+};
+__global__ __launch_bounds__(256) void k_convert_tris(const uint32_t *__restrict__ raw, uint32_t n,
+                                                      float4 *__restrict__ out, TriBounds *__restrict__ bounds) {
+  __shared__ uint32_t s_t[kConvertTris * 25];
+  __shared__ TriBounds s_b[kConvertTris];
+  const uint32_t t = threadIdx.x;
+  TriBounds B;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    B.lo[k] = B.clo[k] = FLT_MAX;
+    B.hi[k] = B.chi[k] = -FLT_MAX;
+  }
+  B.mat_lo = INT32_MAX;
+  B.mat_hi = INT32_MIN;
+  for (uint32_t i0 = blockIdx.x * kConvertTris; i0 < n; i0 += gridDim.x * kConvertTris) {
+    const uint32_t m = min(kConvertTris, n - i0);
+    for (uint32_t i = t; i < 25u * m; i += blockDim.x) s_t[i] = raw[(size_t)25u * i0 + i];
+    __syncthreads();
+    // float4 v of triangle i: a (w: material), b, c, na, nb, nc, (ta, tb), (tc)
+    for (uint32_t q = t; q < 8u * m; q += blockDim.x) {
+      const uint32_t *r = s_t + 25u * (q >> 3);
+      const uint32_t v = q & 7u;
+      float4 f;
+      if (v < 6u)
+        f = make_float4(bitsf(r[3u * v]), bitsf(r[3u * v + 1]), bitsf(r[3u * v + 2]), v == 0u ? bitsf(r[24]) : 0.f);
+      else if (v == 6u) f = make_float4(bitsf(r[18]), bitsf(r[19]), bitsf(r[20]), bitsf(r[21]));
+      else f = make_float4(bitsf(r[22]), bitsf(r[23]), 0.f, 0.f);
+      out[(size_t)8u * i0 + q] = f;
+    }
+    if (t < m) {
+      const uint32_t *r = s_t + 25u * t;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const float a = bitsf(r[k]), b = bitsf(r[3 + k]), c = bitsf(r[6 + k]);
+        B.lo[k] = smin(B.lo[k], smin(a, smin(b, c)));
+        B.hi[k] = smax(B.hi[k], smax(a, smax(b, c)));
+        const float cen = (a + b + c) * (1.0f / 3.0f);
+        B.clo[k] = smin(B.clo[k], cen);
+        B.chi[k] = smax(B.chi[k], cen);
+      }
+      B.mat_lo = min(B.mat_lo, (int32_t)r[24]);
+      B.mat_hi = max(B.mat_hi, (int32_t)r[24]);
+    }
+    __syncthreads();
+  }
+  if (t < kConvertTris) s_b[t] = B;
+  for (uint32_t h = kConvertTris / 2; h > 0; h >>= 1) {
+    __syncthreads();
+    if (t < h) {
+      const TriBounds &o = s_b[t + h];
+      TriBounds &x = s_b[t];
+      for (int k = 0; k < 3; ++k) {
+        x.lo[k] = smin(x.lo[k], o.lo[k]);
+        x.hi[k] = smax(x.hi[k], o.hi[k]);
+        x.clo[k] = smin(x.clo[k], o.clo[k]);
+        x.chi[k] = smax(x.chi[k], o.chi[k]);
+      }
+      x.mat_lo = min(x.mat_lo, o.mat_lo);
+      x.mat_hi = max(x.mat_hi, o.mat_hi);
+    }
+  }
+  if (t == 0) bounds[blockIdx.x] = s_b[0];
+}
+
+// The triangles' boxes for the host builder, in its order of operations.
+__global__ __launch_bounds__(256) void k_tri_boxes(const ShadeTri *__restrict__ tris, uint32_t n,
+                                                   TriBox *__restrict__ out) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const float4 v[3] = {tris[i].a, tris[i].b, tris[i].c};
+  TriBox B;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    B.lo[k] = FLT_MAX;
+    B.hi[k] = -FLT_MAX;
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const float p[3] = {v[c].x, v[c].y, v[c].z};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      B.lo[k] = smin(B.lo[k], p[k]);
+      B.hi[k] = smax(B.hi[k], p[k]);
+    }
+  }
+  out[i] = B;
+}
+
 // Per-pass queue counters: count[0] = all slots, everything else zero.
 // A kernel rather than a memset so the sequence can sit in a hipGraph.
 __global__ void k_pass_setup(const PassDesc *__restrict__ pass, uint32_t *__restrict__ counters, int32_t n) {
@@ -2023,8 +2122,18 @@ struct DBuf {
     if (e == hipSuccess) bytes = std::max<size_t>(n, 256);
     return e;
   }
+  void release() {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    bytes = 0;
+  }
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
+
+// Scratch of scene builds that a context keeps for its next one (triangle
+// staging, device BVH builds: 0.4 KB a triangle); larger blocks are freed
+// after the build.
+constexpr size_t kKeptBuildBytes = (size_t)256 << 20;
 
 }  // namespace
 
@@ -2075,8 +2184,7 @@ struct gi_ctx {
   size_t lds_per_cu = 160 * 1024;
   hipStream_t stream = nullptr;
   std::string err;
-  // scene
-  std::vector<gi_tri> tris;
+  // scene (the triangles live in d_stris; the host builder reads them back)
   std::vector<gi_material> mats;
   std::vector<gi_light> lights;
   std::unique_ptr<gi_bvh> bvh;
@@ -2085,6 +2193,7 @@ struct gi_ctx {
   bool have_bvh = false;
   float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, diag = 0.f, power_total = 0.f;
   float clo[3] = {0, 0, 0}, chi[3] = {0, 0, 0};  // bounds of the triangle centroids
+  DBuf d_build;  // scratch of triangle uploads and device builds
   DBuf d_stris, d_itris, d_nodes, d_hnodes, d_mats, d_lights;  // d_hnodes: HalfNode copy of d_nodes
   DBuf d_ks;  // specular colour per material (float4), for GI_FLAG_PHONG
   DBuf d_lsum;  // running sums of the light powers (n_lights + 1 floats)
@@ -2311,15 +2420,18 @@ int ensure_halton(gi_ctx *ctx, uint32_t seed, int32_t ndims) {
   std::vector<uint16_t> perms;
   uint32_t entries = 0;
   halton_tables(seed, ndims, dims, perms, entries);
-  DBuf d_perms;
-  GI_HIP(ctx, d_perms.ensure(perms.size() * sizeof(uint16_t)));
-  GI_HIP(ctx, ctx->d_hdims.ensure(dims.size() * sizeof(HaltonDim)));
-  GI_HIP(ctx, ctx->d_hchunks.ensure(entries * sizeof(uint16_t)));
+  // the records, then the digit permutations: one buffer, one copy
+  const size_t db = dims.size() * sizeof(HaltonDim);
+  std::vector<uint8_t> up(db + perms.size() * sizeof(uint16_t));
+  std::memcpy(up.data(), dims.data(), db);
+  std::memcpy(up.data() + db, perms.data(), perms.size() * sizeof(uint16_t));
   ctx->hal_dims = 0;  // the old tables are gone from here on
-  GI_HIP(ctx, copy_sync(ctx, ctx->d_hdims.p, dims.data(), dims.size() * sizeof(HaltonDim), hipMemcpyHostToDevice));
-  GI_HIP(ctx, copy_sync(ctx, d_perms.p, perms.data(), perms.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  GI_HIP(ctx, ctx->d_hdims.ensure(up.size()));
+  GI_HIP(ctx, ctx->d_hchunks.ensure(entries * sizeof(uint16_t)));
+  GI_HIP(ctx, hipMemcpyAsync(ctx->d_hdims.p, up.data(), up.size(), hipMemcpyHostToDevice, ctx->stream));
   hipLaunchKernelGGL(halton_fill, dim3(64, (uint32_t)ndims), dim3(256), 0, ctx->stream, ctx->d_hdims.as<HaltonDim>(),
-                     d_perms.as<uint16_t>(), ctx->d_hchunks.as<uint16_t>());
+                     reinterpret_cast<const uint16_t *>(ctx->d_hdims.as<uint8_t>() + db),
+                     ctx->d_hchunks.as<uint16_t>());
   GI_HIP(ctx, hipGetLastError());
   GI_HIP(ctx, hipStreamSynchronize(ctx->stream));
   ctx->hal_seed = seed;
@@ -3382,38 +3494,45 @@ int gi_upload_triangles(gi_ctx *ctx, const gi_tri *tris, int64_t n) {
   if (!ctx || !tris || n <= 0) return fail(ctx, GI_ERR_INVALID_ARG, "triangles");
   if (n > (int64_t)kMaxLeafFirst) return fail(ctx, GI_ERR_LIMIT, "more than 2^27 triangles");
   GI_HIP(ctx, hipSetDevice(ctx->device));
-  ctx->tris.assign(tris, tris + n);
-  ctx->ntri = n;
+  ctx->ntri = 0;
   ctx->have_bvh = false;
   ctx->bvh.reset();
   ctx->meshes.clear();  // a new scene: meshes and instances are uploaded again
   ctx->n_inst = 0;
+  // the records go up as they are and are converted on the device: 1.3 ms
+  // for 291k triangles and 8.6 ms for 2.1M, where the host loop with its
+  // copies and first touches took 10.7 and 74 ms
+  const uint32_t grid = (uint32_t)std::min<int64_t>((n + kConvertTris - 1) / kConvertTris, 1024);
+  const size_t raw = ((size_t)n * sizeof(gi_tri) + 255) & ~(size_t)255;
+  std::vector<TriBounds> part(grid);
+  GI_HIP(ctx, ctx->d_build.ensure(raw + grid * sizeof(TriBounds)));
+  GI_HIP(ctx, ctx->d_stris.ensure(n * sizeof(ShadeTri)));
+  TriBounds *d_part = reinterpret_cast<TriBounds *>(ctx->d_build.as<uint8_t>() + raw);
+  GI_HIP(ctx, copy_sync(ctx, ctx->d_build.p, tris, (size_t)n * sizeof(gi_tri), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(k_convert_tris, dim3(grid), dim3(256), 0, ctx->stream, ctx->d_build.as<uint32_t>(), (uint32_t)n,
+                     ctx->d_stris.as<float4>(), d_part);
+  GI_HIP(ctx, hipGetLastError());
+  GI_HIP(ctx, copy_sync(ctx, part.data(), d_part, grid * sizeof(TriBounds), hipMemcpyDeviceToHost));
+  if (ctx->d_build.bytes > kKeptBuildBytes) ctx->d_build.release();
   ctx->mat_lo = INT32_MAX;
   ctx->mat_hi = INT32_MIN;
-  for (int64_t i = 0; i < n; ++i) {
-    ctx->mat_lo = std::min(ctx->mat_lo, tris[i].material_index);
-    ctx->mat_hi = std::max(ctx->mat_hi, tris[i].material_index);
-  }
   for (int k = 0; k < 3; ++k) {
     ctx->lo[k] = ctx->clo[k] = FLT_MAX;
     ctx->hi[k] = ctx->chi[k] = -FLT_MAX;
   }
-  std::vector<ShadeTri> st(n);
-  for (int64_t i = 0; i < n; ++i) {
-    const gi_tri &t = tris[i];
+  for (const TriBounds &b : part) {
     for (int k = 0; k < 3; ++k) {
-      ctx->lo[k] = std::min(ctx->lo[k], std::min(t.a[k], std::min(t.b[k], t.c[k])));
-      ctx->hi[k] = std::max(ctx->hi[k], std::max(t.a[k], std::max(t.b[k], t.c[k])));
-      const float cen = (t.a[k] + t.b[k] + t.c[k]) * (1.0f / 3.0f);
-      ctx->clo[k] = std::min(ctx->clo[k], cen);
-      ctx->chi[k] = std::max(ctx->chi[k], cen);
+      ctx->lo[k] = std::min(ctx->lo[k], b.lo[k]);
+      ctx->hi[k] = std::max(ctx->hi[k], b.hi[k]);
+      ctx->clo[k] = std::min(ctx->clo[k], b.clo[k]);
+      ctx->chi[k] = std::max(ctx->chi[k], b.chi[k]);
     }
-    st[i] = make_shadetri(t);
+    ctx->mat_lo = std::min(ctx->mat_lo, b.mat_lo);
+    ctx->mat_hi = std::max(ctx->mat_hi, b.mat_hi);
   }
   float dx = ctx->hi[0] - ctx->lo[0], dy = ctx->hi[1] - ctx->lo[1], dz = ctx->hi[2] - ctx->lo[2];
   ctx->diag = std::sqrt(dx * dx + dy * dy + dz * dz);
-  GI_HIP(ctx, ctx->d_stris.ensure(n * sizeof(ShadeTri)));
-  GI_HIP(ctx, copy_sync(ctx, ctx->d_stris.p, st.data(), n * sizeof(ShadeTri), hipMemcpyHostToDevice));
+  ctx->ntri = n;
   return GI_OK;
 }
 
@@ -3537,10 +3656,21 @@ int gi_upload_sky(gi_ctx *ctx, const float *rgb, int32_t w, int32_t h) {
 }
 
 int gi_build_bvh(gi_ctx *ctx, int32_t max_leaf) {
-  if (!ctx || ctx->tris.empty()) return fail(ctx, GI_ERR_STATE, "upload triangles first");
+  if (!ctx || ctx->ntri <= 0) return fail(ctx, GI_ERR_STATE, "upload triangles first");
   GI_HIP(ctx, hipSetDevice(ctx->device));
+  // the builder reads the triangles' boxes only: 24 bytes each come back
+  const size_t n = (size_t)ctx->ntri;
+  std::unique_ptr<TriBox[]> boxes(new (std::nothrow) TriBox[n]);
+  if (!boxes) return fail(ctx, GI_ERR_OUT_OF_MEMORY, "host memory for the triangles' boxes");
+  GI_HIP(ctx, ctx->d_build.ensure(n * sizeof(TriBox)));
+  hipLaunchKernelGGL(k_tri_boxes, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, ctx->stream,
+                     ctx->d_stris.as<ShadeTri>(), (uint32_t)n, ctx->d_build.as<TriBox>());
+  GI_HIP(ctx, hipGetLastError());
+  GI_HIP(ctx, copy_sync(ctx, boxes.get(), ctx->d_build.p, n * sizeof(TriBox), hipMemcpyDeviceToHost));
+  if (ctx->d_build.bytes > kKeptBuildBytes) ctx->d_build.release();
   ctx->bvh = std::make_unique<gi_bvh>();
-  build_bvh2(ctx->tris.data(), (int64_t)ctx->tris.size(), max_leaf > 0 ? max_leaf : 4, *ctx->bvh);
+  build_bvh2(boxes.get(), (int64_t)n, max_leaf > 0 ? max_leaf : 4, *ctx->bvh);
+  boxes.reset();
   return upload_wide(ctx);
 }
 
@@ -3549,7 +3679,7 @@ int gi_build_bvh_device(gi_ctx *ctx, int32_t max_leaf) {
 }
 
 int gi_build_bvh_device_ex(gi_ctx *ctx, int32_t max_leaf, int32_t method, int32_t radius) {
-  if (!ctx || ctx->tris.empty()) return fail(ctx, GI_ERR_STATE, "upload triangles first");
+  if (!ctx || ctx->ntri <= 0) return fail(ctx, GI_ERR_STATE, "upload triangles first");
   const int ml = max_leaf > 0 ? max_leaf : 4;
   if (ml > kMaxLeafTris) return fail(ctx, GI_ERR_INVALID_ARG, "max_leaf must be at most 15");
   if (method != GI_BVH_LBVH && method != GI_BVH_PLOC && method != GI_BVH_SAH)
@@ -3569,8 +3699,15 @@ int gi_build_bvh_device_ex(gi_ctx *ctx, int32_t max_leaf, int32_t method, int32_
                         method == GI_BVH_PLOC  ? DeviceBvhMethod::kPloc
                         : method == GI_BVH_SAH ? DeviceBvhMethod::kSah
                                                : DeviceBvhMethod::kLbvh,
-                        rad, ctx->tuning.node_width, ctx->d_nodes.as<WideNode>(), ctx->d_itris.as<float4>(), r, err))
+                        rad, ctx->tuning.node_width, ctx->d_nodes.as<WideNode>(), ctx->d_itris.as<float4>(),
+                        [ctx](size_t bytes) -> void * {
+                          return ctx->d_build.ensure(bytes) == hipSuccess ? ctx->d_build.p : nullptr;
+                        },
+                        r, err)) {
+    ctx->d_build.release();
     return fail(ctx, GI_ERR_HIP, err);
+  }
+  if (ctx->d_build.bytes > kKeptBuildBytes) ctx->d_build.release();
   return finish_bvh(ctx, r.nnodes, r.depth);
 }
 
@@ -3891,11 +4028,11 @@ int gi_upload_instances(gi_ctx *ctx, const gi_instance *inst, int32_t n) {
 int gi_upload_bvh2(gi_ctx *ctx, const float *nodes, int64_t n_nodes, const uint32_t *indices, int64_t n_indices) {
   if (!ctx || !nodes || n_nodes <= 0 || (!indices && n_indices > 0) || n_indices < 0)
     return fail(ctx, GI_ERR_INVALID_ARG, "bvh2 arrays");
-  if (ctx->tris.empty()) return fail(ctx, GI_ERR_STATE, "upload triangles first");
+  if (ctx->ntri <= 0) return fail(ctx, GI_ERR_STATE, "upload triangles first");
   GI_HIP(ctx, hipSetDevice(ctx->device));
   auto b = std::make_unique<gi_bvh>();
   std::string err;
-  if (!import_bvh2(nodes, n_nodes, indices, n_indices, (int64_t)ctx->tris.size(), *b, err))
+  if (!import_bvh2(nodes, n_nodes, indices, n_indices, ctx->ntri, *b, err))
     return fail(ctx, GI_ERR_INVALID_ARG, err);
   ctx->bvh = std::move(b);
   return upload_wide(ctx);

@@ -248,3 +248,35 @@ def test_image_readback_sizes(w, h, oracle, gpu_ctx_factory):
         out = np.zeros(3 * w * h + 1, np.float32)
         assert ctx.lib.gi_get_image(ctx.h, 0, ptr(out[1:])) == 0
         assert (out[1:].reshape(-1, 3) == ref).all() and out[0] == 0
+
+
+@pytest.mark.parametrize("builder", ["host", "sah", "device", "ploc"])
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 3000, 131_200])
+def test_triangle_upload_sizes(n, builder, oracle, gpu_ctx_factory):
+    """Triangle tables around the upload's blocks (128 triangles, 1024
+    blocks), each replacing the one before: hits, and an image whose ray
+    offsets come from the scene's bounds, are the oracle's."""
+    def soup(n, seed):
+        rng = np.random.default_rng(seed)
+        t = np.zeros(n, scenes.TRI)
+        c = rng.uniform(-5, 5, (n, 3))
+        for k in "abc":
+            t[k] = c + rng.normal(scale=0.3, size=(n, 3))
+            t["n" + k] = rng.normal(size=3)
+            t["t" + k] = rng.uniform(size=(n, 2))
+        t["material_index"] = rng.integers(0, 3, n)
+        view = scenes.make_view((0, 0, -14), (0, 0, 0), (0, 1, 0), 50.0, 24, 16, 2)
+        mats = np.concatenate([scenes.lambert(rng.uniform(0.2, 0.8, 3)) for _ in range(3)])
+        light = scenes.make_light((0, 9, 0), (0, -1, 0), (30, 30, 30), 4, 4)
+        return scenes.Scene(t, mats, light, view, scenes.make_opts(3))
+
+    with gpu_ctx_factory() as ctx:
+        for sc in (soup(500, 1), soup(n, n)):
+            ctx.upload(sc, builder=builder)
+        osc = oracle.OracleScene(sc.tris, sc.mats, sc.lights)
+        assert (ctx.render().image(0).reshape(-1, 3) == osc.render(sc.views, sc.opts)[0]).all()
+        rng = np.random.default_rng(9)
+        o = rng.uniform(-6, 6, (2000, 3)).astype(np.float32)
+        d = rng.normal(size=(2000, 3)).astype(np.float32)
+        t = np.full(2000, np.finfo(np.float32).max, np.float32)
+        assert (ctx.trace_closest(o, d, t) == osc.trace_closest(o, d, t)).all()
