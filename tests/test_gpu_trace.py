@@ -150,6 +150,21 @@ def test_deep_stacks(stack_lds, block, instanced, oracle, gpu_ctx_factory):
         assert ((ctx.trace_any(o, d, t) != 0) == (ref["ref"] != 0xFFFFFFFF)).all()
 
 
+@pytest.mark.parametrize("n", [1, 255, 16383, 16384, 16385])
+def test_host_trace_sizes(n, terrain, oracle, gpu_ctx_factory):
+    """Calls on host arrays around the largest one that goes through pinned
+    memory (16384 rays): hits and occlusion of each call are the oracle's."""
+    osc = oracle.OracleScene(terrain.tris)
+    rng = np.random.default_rng(n)
+    with gpu_ctx_factory(terrain) as ctx:
+        for _ in range(2):
+            o, d = _rays(rng, n, -5, 105, 0, 20)
+            t = np.where(rng.random(n) < 0.5, rng.uniform(0, 30, n), FMAX).astype(np.float32)
+            ref = osc.trace_closest(o, d, t)
+            _assert_hits_equal(ctx.trace_closest(o, d, t), ref, osc, o, d, t)
+            assert ((ctx.trace_any(o, d, t) != 0) == (ref["ref"] != 0xFFFFFFFF)).all()
+
+
 def test_call_order_and_argument_errors(c1, gpu_ctx_factory):
     with gpu_ctx_factory() as ctx:
         with pytest.raises(GiError) as e:
