@@ -2294,23 +2294,23 @@ constexpr uint32_t kStagePixels = (uint32_t)(kStageBytes / 12);
 // blocks are kept for the process's next read-backs, on any thread and
 // device, until its last context is destroyed.
 std::mutex g_stage_mu;
-std::vector<uint8_t *> g_stage_free;
+constexpr int kStageKept = 2;
+uint8_t *g_stage_free[kStageKept];
+int g_stage_nfree = 0;
 int g_stage_contexts = 0;
 void stage_contexts(int change) {
   std::lock_guard<std::mutex> lock(g_stage_mu);
   g_stage_contexts += change;
   if (g_stage_contexts > 0) return;
-  for (uint8_t *p : g_stage_free) (void)hipHostFree(p);
-  g_stage_free.clear();
+  while (g_stage_nfree > 0) (void)hipHostFree(g_stage_free[--g_stage_nfree]);
 }
 struct StageLease {
   uint8_t *p = nullptr;
   hipError_t take() {
     {
       std::lock_guard<std::mutex> lock(g_stage_mu);
-      if (!g_stage_free.empty()) {
-        p = g_stage_free.back();
-        g_stage_free.pop_back();
+      if (g_stage_nfree > 0) {
+        p = g_stage_free[--g_stage_nfree];
         return hipSuccess;
       }
     }
@@ -2322,7 +2322,7 @@ struct StageLease {
   ~StageLease() {
     if (!p) return;
     std::lock_guard<std::mutex> lock(g_stage_mu);
-    if (g_stage_free.size() < 2) g_stage_free.push_back(p);
+    if (g_stage_nfree < kStageKept) g_stage_free[g_stage_nfree++] = p;
     else (void)hipHostFree(p);
   }
 };
@@ -4369,18 +4369,18 @@ int gi_get_image(gi_ctx *ctx, int32_t view, float *rgb) {
     }
   };
   for (int s = 0; s < workers; ++s) launch(s, (size_t)s);
-  std::vector<std::thread> pool;
-  std::vector<int> left;  // slots whose thread could not start
+  std::thread pool[kStageSlots];
   for (int s = 1; s < workers; ++s) {
     try {
-      pool.emplace_back(work, s);
-    } catch (const std::exception &) {
-      left.push_back(s);
+      pool[s] = std::thread(work, s);
+    } catch (const std::exception &) {  // no thread to be had: this one does the slot below
     }
   }
   work(0);
-  for (int s : left) work(s);
-  for (std::thread &t : pool) t.join();
+  for (int s = 1; s < workers; ++s) {
+    if (pool[s].joinable()) pool[s].join();
+    else work(s);
+  }
   GI_HIP(ctx, hipStreamSynchronize(ctx->stream));  // nothing reads the slots or the image after the return
   GI_HIP(ctx, (hipError_t)err.load());
   return GI_OK;
