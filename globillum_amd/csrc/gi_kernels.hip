@@ -2315,7 +2315,9 @@ struct StageLease {
       }
     }
     void *q = nullptr;
-    const hipError_t e = hipHostMalloc(&q, kStageSlots * kStageBytes, hipHostMallocPortable);
+    // coherent by flag: kernels write here and the host reads after an event
+    const hipError_t e =
+        hipHostMalloc(&q, kStageSlots * kStageBytes, hipHostMallocPortable | hipHostMallocCoherent);
     p = static_cast<uint8_t *>(q);
     return e;
   }

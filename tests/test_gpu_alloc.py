@@ -1,0 +1,73 @@
+"""What the library asks of the HIP allocator, and what it does when it is
+refused: each case runs in a process of its own, behind tests/csrc/
+hip_alloc_stub.cpp, which passes the calls on and refuses sizes above a
+limit on request."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes as C, sys
+stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+class S:
+    def __getattr__(self, k): return C.c_uint64.in_dll(stub, "stub_" + k).value
+    def __setattr__(self, k, v): C.c_uint64.in_dll(stub, "stub_" + k).value = v
+S = S()
+flags_all = lambda: C.c_uint32.in_dll(stub, "stub_pinned_flags_all").value
+import numpy as np
+from globillum_amd import scenes
+from globillum_amd._lib import GiError
+from globillum_amd.context import Context
+import pyoracle as oracle
+FMAX = np.finfo(np.float32).max
+def rays(n, seed=1):
+    rng = np.random.default_rng(seed)
+    return (rng.uniform(-0.9, 0.9, (n, 3)).astype(np.float32), rng.normal(size=(n, 3)).astype(np.float32),
+            np.full(n, FMAX, np.float32))
+def same_image(ctx, sc):
+    ref, _ = oracle.OracleScene(sc.tris, sc.mats, sc.lights).render(sc.views, sc.opts)
+    assert (ctx.render().image(0).reshape(-1, 3) == ref).all()
+def same_hits(ctx, sc, n, seed=1):
+    o, d, t = rays(n, seed)
+    osc = oracle.OracleScene(sc.tris)
+    ref = osc.trace_closest(o, d, t)
+    assert (ctx.trace_closest(o, d, t) == ref).all()
+    assert ((ctx.trace_any(o, d, t) != 0) == (ref["ref"] != 0xFFFFFFFF)).all()
+"""
+
+
+@pytest.fixture(scope="module")
+def child(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("stub") / "alloc_stub.so")
+    cxx = shutil.which("g++") or "g++"
+    r = subprocess.run([cxx, "-O1", "-std=c++17", "-shared", "-fPIC", "-o", so,
+                        os.path.join(ROOT, "tests", "csrc", "hip_alloc_stub.cpp"), "-ldl"],
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+
+    def run(body):
+        env = dict(os.environ, PYTHONPATH=os.pathsep.join([ROOT, os.path.join(ROOT, "oracle")]))
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, so], capture_output=True, text=True, timeout=100,
+                           env=env, cwd=ROOT)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return run
+
+
+def test_pinned_memory_is_coherent(child):
+    """Kernels write results straight into the pinned blocks and the host
+    reads them after an event: that needs coherent memory, which the calls
+    ask for by flag (hipHostMallocCoherent) and leave to no default."""
+    child("""
+sc = scenes.cornell_boxes(w=64, h=48, spp=2, depth=3)
+with Context(0).upload(sc) as ctx:
+    same_hits(ctx, sc, 1000)
+    same_image(ctx, sc)
+assert S.pinned > 0 and flags_all() & 0x40000000, (S.pinned, hex(flags_all()))
+""")
