@@ -2306,20 +2306,23 @@ void stage_contexts(int change) {
 }
 struct StageLease {
   uint8_t *p = nullptr;
-  hipError_t take() {
+  // false: the runtime has no pinned memory left (the caller goes by pageable copies)
+  bool take() {
     {
       std::lock_guard<std::mutex> lock(g_stage_mu);
       if (g_stage_nfree > 0) {
         p = g_stage_free[--g_stage_nfree];
-        return hipSuccess;
+        return true;
       }
     }
     void *q = nullptr;
     // coherent by flag: kernels write here and the host reads after an event
-    const hipError_t e =
-        hipHostMalloc(&q, kStageSlots * kStageBytes, hipHostMallocPortable | hipHostMallocCoherent);
+    if (hipHostMalloc(&q, kStageSlots * kStageBytes, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();  // the refusal is not the next launch's error
+      return false;
+    }
     p = static_cast<uint8_t *>(q);
-    return e;
+    return true;
   }
   ~StageLease() {
     if (!p) return;
@@ -4135,17 +4138,24 @@ namespace {
 constexpr int64_t kPinnedTraceRays = 16384;
 static_assert((28 + 16) * kPinnedTraceRays + 64 <= (int64_t)(kStageSlots * kStageBytes), "the block holds a call's rays");
 
+// The block and the packed rays' buffers; false: one of them is not to be had
+// (the call goes by copies, which need no block and smaller buffers).
+bool pinned_trace_ready(gi_ctx *ctx, StageLease &stage) {
+  if (hipSetDevice(ctx->device) != hipSuccess || !stage.take()) return false;
+  if (ctx->p_ro.ensure(kPinnedTraceRays * sizeof(float4)) == hipSuccess &&
+      ctx->p_rd.ensure(kPinnedTraceRays * sizeof(float4)) == hipSuccess)
+    return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 // out: n gi_hit (closest) or n bytes (any).  About 30 us for a thousand rays
 // on a small scene, where three copies, a clear, two waits and a copy back
 // took 117 us.
-int trace_pinned(gi_ctx *ctx, bool any, const float *orig, const float *dir, const float *max_t, int64_t n, void *out) {
-  GI_HIP(ctx, hipSetDevice(ctx->device));
+int trace_pinned(gi_ctx *ctx, StageLease &stage, bool any, const float *orig, const float *dir, const float *max_t,
+                 int64_t n, void *out) {
   int rc = ensure_gstack(ctx);
   if (rc) return rc;
-  GI_HIP(ctx, ctx->p_ro.ensure(kPinnedTraceRays * sizeof(float4)));
-  GI_HIP(ctx, ctx->p_rd.ensure(kPinnedTraceRays * sizeof(float4)));
-  StageLease stage;
-  GI_HIP(ctx, stage.take());
   const size_t c = (size_t)n, res = c * (any ? 1 : sizeof(gi_hit));
   uint8_t *hits = stage.p;  // 16-byte aligned
   uint32_t *overflow = reinterpret_cast<uint32_t *>(stage.p + ((res + 15) & ~(size_t)15));
@@ -4180,7 +4190,10 @@ int gi_trace_closest(gi_ctx *ctx, const float *orig, const float *dir, const flo
   if (rc) return rc;
   if (n < 0 || (n > 0 && (!orig || !dir || !max_t || !out))) return fail(ctx, GI_ERR_INVALID_ARG, "rays");
   if (n == 0) return GI_OK;
-  if (n <= kPinnedTraceRays) return trace_pinned(ctx, false, orig, dir, max_t, n, out);
+  if (n <= kPinnedTraceRays) {
+    StageLease stage;
+    if (pinned_trace_ready(ctx, stage)) return trace_pinned(ctx, stage, false, orig, dir, max_t, n, out);
+  }
   GI_HIP(ctx, hipSetDevice(ctx->device));
   GI_HIP(ctx, ctx->p_orig.ensure(n * 12));
   GI_HIP(ctx, ctx->p_dir.ensure(n * 12));
@@ -4201,7 +4214,10 @@ int gi_trace_any(gi_ctx *ctx, const float *orig, const float *dir, const float *
   if (rc) return rc;
   if (n < 0 || (n > 0 && (!orig || !dir || !max_t || !occluded))) return fail(ctx, GI_ERR_INVALID_ARG, "rays");
   if (n == 0) return GI_OK;
-  if (n <= kPinnedTraceRays) return trace_pinned(ctx, true, orig, dir, max_t, n, occluded);
+  if (n <= kPinnedTraceRays) {
+    StageLease stage;
+    if (pinned_trace_ready(ctx, stage)) return trace_pinned(ctx, stage, true, orig, dir, max_t, n, occluded);
+  }
   GI_HIP(ctx, hipSetDevice(ctx->device));
   GI_HIP(ctx, ctx->p_orig.ensure(n * 12));
   GI_HIP(ctx, ctx->p_dir.ensure(n * 12));
@@ -4327,6 +4343,26 @@ int gi_progress_step(gi_ctx *ctx, int32_t *done) {
   return GI_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// The read-back without pinned memory: the float4 image as it is, then its
+// colours in a loop.
+int get_image_copied(gi_ctx *ctx, int32_t view, size_t npix, float *rgb) {
+  std::unique_ptr<float4[]> tmp(new (std::nothrow) float4[npix]);
+  if (!tmp) return fail(ctx, GI_ERR_OUT_OF_MEMORY, "host memory for the image");
+  GI_HIP(ctx, copy_sync(ctx, tmp.get(), ctx->images[view].p, npix * sizeof(float4), hipMemcpyDeviceToHost));
+  for (size_t i = 0; i < npix; ++i) {
+    rgb[3 * i] = tmp[i].x;
+    rgb[3 * i + 1] = tmp[i].y;
+    rgb[3 * i + 2] = tmp[i].z;
+  }
+  return GI_OK;
+}
+}  // namespace
+
+extern "C" {
+
 int gi_get_image(gi_ctx *ctx, int32_t view, float *rgb) {
   if (!ctx || !rgb) return fail(ctx, GI_ERR_INVALID_ARG, "get_image");
   if (view < 0 || view >= (int32_t)ctx->views.size()) return fail(ctx, GI_ERR_INVALID_ARG, "view index");
@@ -4335,9 +4371,13 @@ int gi_get_image(gi_ctx *ctx, int32_t view, float *rgb) {
   const size_t chunks = (npix + kStagePixels - 1) / kStagePixels;
   const int workers = (int)std::min<size_t>(chunks, kStageSlots);
   StageLease stage;
-  GI_HIP(ctx, stage.take());
-  for (int s = 0; s < workers; ++s)
-    if (!ctx->stage_ev[s]) GI_HIP(ctx, hipEventCreateWithFlags(&ctx->stage_ev[s], hipEventDisableTiming));
+  bool staged = stage.take();
+  for (int s = 0; s < workers && staged; ++s)
+    if (!ctx->stage_ev[s]) staged = hipEventCreateWithFlags(&ctx->stage_ev[s], hipEventDisableTiming) == hipSuccess;
+  if (!staged) {
+    (void)hipGetLastError();
+    return get_image_copied(ctx, view, npix, rgb);
+  }
   // The image goes over in chunks: a kernel packs a chunk into a pinned slot
   // over the bus, a host thread copies the slot to the caller's memory.  The
   // chunk of a slot is launched again as soon as the slot's copy is done, so

@@ -25,6 +25,7 @@ from globillum_amd import scenes
 from globillum_amd._lib import GiError
 from globillum_amd.context import Context
 import pyoracle as oracle
+from test_gpu_trace import _assert_hits_equal
 FMAX = np.finfo(np.float32).max
 def rays(n, seed=1):
     rng = np.random.default_rng(seed)
@@ -37,7 +38,7 @@ def same_hits(ctx, sc, n, seed=1):
     o, d, t = rays(n, seed)
     osc = oracle.OracleScene(sc.tris)
     ref = osc.trace_closest(o, d, t)
-    assert (ctx.trace_closest(o, d, t) == ref).all()
+    _assert_hits_equal(ctx.trace_closest(o, d, t), ref, osc, o, d, t)
     assert ((ctx.trace_any(o, d, t) != 0) == (ref["ref"] != 0xFFFFFFFF)).all()
 """
 
@@ -52,7 +53,7 @@ def child(tmp_path_factory):
     assert r.returncode == 0, r.stderr
 
     def run(body):
-        env = dict(os.environ, PYTHONPATH=os.pathsep.join([ROOT, os.path.join(ROOT, "oracle")]))
+        env = dict(os.environ, PYTHONPATH=os.pathsep.join([ROOT, os.path.join(ROOT, "oracle"), os.path.join(ROOT, "tests")]))
         r = subprocess.run([sys.executable, "-c", PRELUDE + body, so], capture_output=True, text=True, timeout=100,
                            env=env, cwd=ROOT)
         assert r.returncode == 0, r.stdout + r.stderr
@@ -70,4 +71,32 @@ with Context(0).upload(sc) as ctx:
     same_hits(ctx, sc, 1000)
     same_image(ctx, sc)
 assert S.pinned > 0 and flags_all() & 0x40000000, (S.pinned, hex(flags_all()))
+""")
+
+
+def test_refused_pinned_memory(child):
+    """Without pinned memory, or without room for the largest pinned call's
+    ray buffers, images and host-array traces go by copies: the same results
+    and no error, also from the calls after the refusal."""
+    child("""
+sc = scenes.cornell_boxes(w=300, h=301, spp=1, depth=3)
+with Context(0).upload(sc) as ctx:
+    S.max_pinned = 0
+    for n in (1, 1000, 16384, 20000):
+        same_hits(ctx, sc, n, n)
+    same_image(ctx, sc)
+    same_image(ctx, sc)
+    assert S.refused > 0 and S.pinned == 0
+    S.max_pinned = 2 ** 64 - 1
+    same_image(ctx, sc)
+    same_hits(ctx, sc, 1000)
+    assert S.pinned > 0
+with Context(0).upload(sc) as ctx:
+    n = S.refused
+    S.max_device = 100000
+    same_hits(ctx, sc, 1000)
+    assert S.refused > n
+    S.max_device = 2 ** 64 - 1
+    same_hits(ctx, sc, 1000, 2)
+    same_image(ctx, sc)
 """)
