@@ -2267,6 +2267,7 @@ namespace {
   do {                                                                             \
     hipError_t e_ = (expr);                                                        \
     if (e_ != hipSuccess) {                                                        \
+      (void)hipGetLastError(); /* reported here: not the next launch's error */    \
       (ctx)->err = std::string(#expr) + ": " + hipGetErrorString(e_);              \
       return e_ == hipErrorOutOfMemory ? GI_ERR_OUT_OF_MEMORY : GI_ERR_HIP;        \
     }                                                                              \
@@ -3713,6 +3714,7 @@ int gi_build_bvh_device_ex(gi_ctx *ctx, int32_t max_leaf, int32_t method, int32_
                         },
                         r, err)) {
     ctx->d_build.release();
+    (void)hipGetLastError();
     return fail(ctx, GI_ERR_HIP, err);
   }
   if (ctx->d_build.bytes > kKeptBuildBytes) ctx->d_build.release();

@@ -100,3 +100,22 @@ with Context(0).upload(sc) as ctx:
     same_hits(ctx, sc, 1000, 2)
     same_image(ctx, sc)
 """)
+
+
+def test_calls_after_a_refused_upload(child):
+    """A texture upload that the device has no memory for fails with that
+    error, once: the calls after it, uploads among them, work as before."""
+    child("""
+sc = scenes.cornell_boxes(w=40, h=30, spp=1, depth=2)
+with Context(0).upload(sc) as ctx:
+    same_hits(ctx, sc, 100)
+    for again in (lambda: same_hits(ctx, sc, 100), lambda: ctx.upload(sc, builder="sah"), lambda: same_image(ctx, sc)):
+        S.max_device = 1 << 20
+        try:
+            ctx.upload_texture(np.zeros((1024, 1024, 4), np.uint8))
+            assert False, "granted"
+        except GiError as e:
+            assert "memory" in str(e), e
+        S.max_device = 2 ** 64 - 1
+        again()
+""")
