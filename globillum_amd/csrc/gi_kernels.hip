@@ -2918,6 +2918,7 @@ int ensure_workspace(gi_ctx *ctx, size_t slots) {
     if (ctx->textured) GI_HIP(ctx, ctx->rdiff.ensure(4 * ctx->slot_cap * sizeof(float4)));
     return GI_OK;
   }
+  ctx->slot_cap = 0;  // a buffer that cannot grow is gone: nothing fits until all have
   // path state by slot; kShards segments of segment_cap entries are at most
   // kShards tiles each longer, whatever the tile (at most 256)
   const size_t p4 = slots * sizeof(float4);

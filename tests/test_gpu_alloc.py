@@ -119,3 +119,26 @@ with Context(0).upload(sc) as ctx:
         S.max_device = 2 ** 64 - 1
         again()
 """)
+
+
+def test_renders_after_a_refused_workspace(child):
+    """A render whose path buffers are refused fails; a smaller one behind it
+    does not run on what the refused growth left (the buffers it had are
+    freed by then)."""
+    child("""
+sc = scenes.cornell_boxes(w=40, h=30, spp=2, depth=2)
+big = scenes.cornell_boxes(w=256, h=256, spp=16, depth=2)
+with Context(0).upload(sc) as ctx:
+    same_image(ctx, sc)
+    S.max_device = 4 << 20
+    try:
+        ctx.render(big.views, big.opts)
+        assert False, "granted"
+    except GiError as e:
+        assert "memory" in str(e), e
+    ref, _ = oracle.OracleScene(sc.tris, sc.mats, sc.lights).render(sc.views, sc.opts)
+    assert (ctx.render(sc.views, sc.opts).image(0).reshape(-1, 3) == ref).all()
+    S.max_device = 2 ** 64 - 1
+    ref, _ = oracle.OracleScene(big.tris, big.mats, big.lights).render(big.views, big.opts)
+    assert (ctx.render(big.views, big.opts).image(0).reshape(-1, 3) == ref).all()
+""")
