@@ -54,13 +54,28 @@ constexpr uint32_t kEmptyRef = 0x80000000u;  // a leaf with zero triangles
 constexpr int kMaxLeafTris = 15;
 constexpr uint32_t kMaxLeafFirst = (1u << 27) - 1;
 
+#if defined(__HIP__)
+#define GI_HOST_DEVICE __host__ __device__
+#else
+#define GI_HOST_DEVICE
+#endif
+
+// The slab tests' relative slack, and their limit: the nearer of the ray's
+// limit and the largest float whose product with the slack is finite.  That
+// product is FLT_MAX, so a ray without a limit reaches every box at a finite
+// distance and no box at +inf.  A limit of NaN counts as none.
+constexpr float kSlabSlack = 1.0f + 0x1p-21f;
+constexpr float kMaxLim = 0x1.ffffeep127f;
+static_assert(kMaxLim * kSlabSlack == 0x1.fffffep127f, "the largest limit stays finite, at FLT_MAX");
+GI_HOST_DEVICE inline float slab_limit(float lim) { return lim < kMaxLim ? lim : kMaxLim; }
+// A box entered at tn (at least 0) and left at tf (at most the limit).
+GI_HOST_DEVICE inline bool slab_hit(float tn, float tf) { return tn <= tf * kSlabSlack; }
+
 // An empty child slot: its box is [+inf, +inf] on every axis, so the slab
 // test never reports it (each plane distance is +inf or -inf for any finite
-// nonzero inverse direction) and the traversal needs no reference check.
-#if defined(__HIP__)
-__host__ __device__
-#endif
-inline void set_empty_slot(WideNode &nd, int k) {
+// nonzero inverse direction: entered at +inf, or left at -inf, both beyond
+// slab_limit) and the traversal needs no reference check.
+GI_HOST_DEVICE inline void set_empty_slot(WideNode &nd, int k) {
   nd.lox[k] = nd.loy[k] = nd.loz[k] = __builtin_inff();
   nd.hix[k] = nd.hiy[k] = nd.hiz[k] = __builtin_inff();
   nd.child[k] = kEmptyRef;

@@ -299,10 +299,6 @@ constexpr uint32_t kNoRay = 0xffffffffu;
 // The traversal addresses a node's planes by a 32-bit byte offset (index
 // << 7): at most 2^25 wide nodes.
 constexpr uint64_t kMaxWideNodes = (uint64_t)1 << 25;
-constexpr float kSlabSlack = 1.0f + 0x1p-21f;
-// The slab tests' limit is finite after the slack too, so that an empty
-// slot (a box at +inf) is never within it.
-constexpr float kMaxLim = 0x1.fffff0p127f;
 // The interior-node loop hands over to the leaf tests once at most this
 // many lanes of the wave are still looking for their first leaf (and some
 // lane holds one): the last searchers would otherwise keep the whole wave
@@ -568,7 +564,7 @@ __device__ __forceinline__ void trace_persistent(QueueIn Q, uint32_t cs, const H
       continue;
     }
     if (ray == kNoRay) continue;
-    const float lim = smin(kMaxLim, kAny ? tmax : smin(bt, tmax));
+    const float lim = slab_limit(kAny ? tmax : smin(bt, tmax));
     const float far = lim * kSlabSlack;  // entries beyond it cannot hold the result
     if constexpr (kDist) {
       // the leaf tests may have brought the limit below the waiting entry
@@ -618,7 +614,7 @@ __device__ __forceinline__ void trace_persistent(QueueIn Q, uint32_t cs, const H
                                    fmaxf(fmaf(nz[k], idir.z, -oid.z), 0.0f));
             const float tf = fminf(fminf(fmaf(fx[k], idir.x, -oid.x), fmaf(fy[k], idir.y, -oid.y)),
                                    fminf(fmaf(fz[k], idir.z, -oid.z), lim));
-            hit[k] = tn <= tf * kSlabSlack;  // empty slots: +inf boxes, never hit
+            hit[k] = slab_hit(tn, tf);  // empty slots: +inf boxes, never hit
             dist[k] = hit[k] ? tn : -1.0f;
           }
         } else {
@@ -647,7 +643,7 @@ __device__ __forceinline__ void trace_persistent(QueueIn Q, uint32_t cs, const H
   {                                                                                                  \
     const float tn = max3_raw(MIX(NX, sx, bx), MIX(NY, sy, by), max3_raw(MIX(NZ, sz, bz), 0.0f, 0.0f)); \
     const float tf = min3_raw(MIX(FX, sx, bx), MIX(FY, sy, by), min3_raw(MIX(FZ, sz, bz), lim, lim));  \
-    hit[k] = tn <= tf * kSlabSlack; /* empty slots: +inf boxes, never hit */                           \
+    hit[k] = slab_hit(tn, tf); /* empty slots: +inf boxes, never hit */                                \
     dist[k] = hit[k] ? tn : -1.0f;                                                                     \
   }
           GI_SLAB(0, nx0, ny0, nz0, fx0, fy0, fz0, mix_lo)

@@ -2,6 +2,10 @@
 Moller-Trumbore against FP64 and known answers, BVH traversal (the
 oracle's own median BVH and the product's binned-SAH BVH) against brute
 force, any-hit against closest hit, and the host BVH's invariants."""
+import os
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -163,3 +167,18 @@ def test_host_bvh_empty_and_errors():
     one["c"] = (0, 1, 0)
     nodes, idx = build_bvh2(one)
     assert len(nodes) == 8 and idx.tolist() == [0]
+
+
+def test_empty_slots_are_never_hit(tmp_path):
+    """The kernels' slab test, compiled for the host from the same header
+    (tests/csrc/slab_check.cpp): empty child slots miss for all eight sign
+    combinations and for limits up to infinity and NaN; boxes at finite
+    distances within the limit hit."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = str(tmp_path / "slab_check")
+    r = subprocess.run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-ffp-contract=off", "-o", exe,
+                        os.path.join(root, "tests", "csrc", "slab_check.cpp")], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stderr
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and " 0 bad" in r.stdout, r.stdout
