@@ -322,11 +322,15 @@ constexpr size_t kLdsSceneMaxBytes = 10240;
 // of its box, so that it can be dropped without a node visit once a hit
 // nearer than it is known.  Of the distance only the upper 16 bits are kept
 // in LDS (rounded towards zero: nothing is dropped too early): 6 bytes an
-// entry, 17 rows at 6 blocks of 256 lanes per CU.  8-byte entries leave 13
+// entry, 16 rows at 6 waves per SIMD.  8-byte entries leave 13
 // rows: 2 % faster on a 291k-triangle tree and 1.3 % slower on the 4.2M-
 // triangle two-level one, whose stacks run past 13 rows more often.
-// LDS layout: the distances (kRows * 512 bytes, for any block size up to
-// 256), then the references, both interleaved by lane (no bank conflicts).
+// LDS layout: the distances, then the references, both interleaved by lane
+// (no bank conflicts) in rows of the next power of two of the block's lanes,
+// so that a block of any size takes 6 bytes an entry and lane (with rows for
+// 256 lanes whatever the block, 12 instead of 24 blocks of 64 fitted a CU: 61
+// instead of 26 ms for the closest hits of a 3840x2160x8 frame of the
+// 4.2M-triangle scene; blocks of 128: 30.5 instead of 26.4 ms).
 // The kernels have no static LDS, so the dynamic LDS starts at address 0 and
 // entries are addressed by 32-bit offsets.  The global columns hold
 // references only; entries from there are never dropped.
@@ -334,21 +338,24 @@ struct StackEntry {
   uint32_t ref;
   float dist;
 };
-constexpr uint32_t stack_dist_bytes(int rows, bool dist) { return dist ? (uint32_t)rows * 512u : 0u; }
 template <int kRows, bool kDist>
 struct Stack {
-  static constexpr uint32_t kRefs = stack_dist_bytes(kRows, kDist);  // LDS address of the references
+  static constexpr uint32_t kUnit = kDist ? 1u : 2u;  // log2 of the bytes from lane to lane of what top addresses
   typedef __attribute__((address_space(3))) uint16_t lds_u16;
-  uint32_t top;    // the lane's next free entry: its reference lies at kRefs + top, the upper half of its distance
-                   // at top / 2 (top goes on counting beyond the LDS rows)
-  uint32_t rsh;    // log2 of the bytes from row to row of the references (wave-uniform)
+  uint32_t top;    // LDS address of the lane's next free entry: with distances, of the upper half of its distance
+                   // (its reference lies at 2 top + refs), else of its reference (top goes on counting beyond the
+                   // LDS rows)
+  uint32_t rsh;    // log2 of the bytes from row to row of what top addresses (wave-uniform)
+  uint32_t refs;   // LDS address of the references (wave-uniform)
   uint32_t *gbase; // the global columns: the reference of entry k of thread t at [(k - kRows) * gstride + t]
   uint32_t gstride;
   uint32_t tid0;   // first thread of the wave (wave-uniform)
   int cap;         // entries the column holds, the sentinel included
-  __device__ __forceinline__ static lds_u32 *ref_at(uint32_t t) { return (lds_u32 *)(uintptr_t)t + kRefs / 4u; }
-  __device__ __forceinline__ static lds_u16 *dist_at(uint32_t t) { return (lds_u16 *)(uintptr_t)(t >> 1); }
-  __device__ __forceinline__ uint32_t bottom() const { return (tid0 + __lane_id()) * 4u; }
+  __device__ __forceinline__ lds_u32 *ref_at(uint32_t t) const {
+    return (lds_u32 *)(uintptr_t)(kDist ? (t << 1) + refs : t);
+  }
+  __device__ __forceinline__ static lds_u16 *dist_at(uint32_t t) { return (lds_u16 *)(uintptr_t)t; }
+  __device__ __forceinline__ uint32_t bottom() const { return (tid0 + __lane_id()) << kUnit; }
   __device__ __forceinline__ uint32_t *column(int k) const {
     return gbase + (size_t)(k - kRows) * gstride + blockIdx.x * blockDim.x + tid0 + __lane_id();
   }
@@ -442,18 +449,23 @@ __device__ __forceinline__ float min3_raw(float a, float b, float c) {
   return r;
 }
 
-// LDS column stride of a block: the next power of two >= blockDim.
-__host__ __device__ __forceinline__ uint32_t lds_shift_for(uint32_t block) {
+// LDS row of a block's stack: the next power of two >= blockDim lanes.
+__host__ __device__ constexpr uint32_t lds_shift_for(uint32_t block) {
   uint32_t s = 0;
   while ((1u << s) < block) ++s;
   return s;
+}
+// LDS bytes of a traversal block's stacks of `rows` entries a lane.
+constexpr size_t trace_lds_bytes(int rows, int block, bool dist) {
+  return ((size_t)rows << lds_shift_for((uint32_t)block)) * (dist ? 6u : 4u);
 }
 
 template <int kRows, bool kDist>
 __device__ __forceinline__ Stack<kRows, kDist> make_stack(uint32_t *smem, uint32_t *gstack, uint32_t cap) {
   const uint32_t shift = blockDim.x <= 1 ? 0u : 32u - (uint32_t)__clz((int)(blockDim.x - 1));
   using S = Stack<kRows, kDist>;
-  return S{0u, shift + 2u, gstack, gridDim.x * blockDim.x,
+  const uint32_t rsh = shift + S::kUnit;
+  return S{0u, rsh, (uint32_t)kRows << rsh, gstack, gridDim.x * blockDim.x,
            (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u)), (int)cap};
 }
 
@@ -824,14 +836,32 @@ __device__ __forceinline__ void trace_persistent(QueueIn Q, uint32_t cs, const H
 
 // LDS rows of the traversal stack (entries per lane, the sentinel and the
 // four rows a push may scratch included) for a tuned depth of 8, 16 or 32;
-// dist: the entries carry distances.  At the default depth of 16, 17 rows
-// with distances and 20 without keep 6 blocks of 256 lanes on a CU; 16
-// without them next to an LDS scene copy (dropping by distance there, in 12
-// rows, was 3 % slower: its visits are cheap).
+// dist: the entries carry distances.  At the default depth of 16, 16 rows
+// with distances and 20 without keep 6 waves per SIMD in blocks of 64, 128
+// and 256 lanes; 16 without them next to an LDS scene copy (dropping by
+// distance there, in 12 rows, was 3 % slower: its visits are cheap).
 __host__ __device__ constexpr int stack_rows(int lds_depth, bool lds_scene, bool dist) {
-  return lds_scene ? 16 : lds_depth == 8 ? 12 : lds_depth == 32 ? 32 : dist ? 17 : 20;
+  return lds_depth == 8 ? 12 : lds_depth == 32 ? 32 : lds_scene || dist ? 16 : 20;
 }
 constexpr int kMinRows = 12;  // smallest instantiated LDS part; sizes the global part
+// The tuned depth whose rows the closest-hit stack takes: blocks of 192
+// lanes have rows of 256, of which 16 would leave 6 instead of 8 on a CU.
+constexpr int closest_depth(int lds_depth, int block) { return lds_depth == 16 && block == 192 ? 8 : lds_depth; }
+// A block's LDS is granted in pieces of this size (measured: 25 blocks of
+// 6400 bytes are resident on a CU, 21 of 6401).
+constexpr size_t kLdsPiece = 1280;
+constexpr size_t lds_granted(size_t bytes) { return (bytes + kLdsPiece - 1) / kLdsPiece * kLdsPiece; }
+// At the default depth the stacks of GI_TRACE_WAVES_PER_EU waves per SIMD,
+// as many as the registers allow, fit the CU's 160 KB for every block size.
+constexpr bool lds_holds_all_waves(int block, bool dist) {
+  const int rows = stack_rows(dist ? closest_depth(16, block) : 16, false, dist);
+  return GI_TRACE_WAVES_PER_EU * 4 / (block / 64) * lds_granted(trace_lds_bytes(rows, block, dist)) <= 160 * 1024;
+}
+static_assert(lds_holds_all_waves(64, true) && lds_holds_all_waves(128, true) && lds_holds_all_waves(192, true) &&
+                  lds_holds_all_waves(256, true) && lds_holds_all_waves(64, false) &&
+                  lds_holds_all_waves(128, false) && lds_holds_all_waves(192, false) &&
+                  lds_holds_all_waves(256, false),
+              "the traversal stacks keep waves off the CU");
 
 // Closest-hit kernel over a ray queue.  kHasTmax: max_t in ray_o.w (the
 // primitive entry point); otherwise ray_o.w carries the Halton index and
@@ -2660,7 +2690,6 @@ int ensure_gstack(gi_ctx *ctx) {
 
 int stack_lds_of(const gi_ctx *ctx);
 bool lds_scene_of(const gi_ctx *ctx);
-size_t trace_lds_bytes(int rows, int block, bool dist);
 
 // Traversal blocks per CU that are resident at once: the tuned count,
 // capped by the waves the register budget allows (GI_TRACE_WAVES_PER_EU per
@@ -2671,9 +2700,11 @@ size_t trace_lds_bytes(int rows, int block, bool dist);
 int resident_trace_blocks(const gi_ctx *ctx, int block, bool closest) {
   const int by_waves = GI_TRACE_WAVES_PER_EU * 4 / std::max(1, block / 64);
   const bool lds_scene = !ctx->count_traversal && stack_lds_of(ctx) == 16 && lds_scene_of(ctx);
-  const size_t lds = trace_lds_bytes(stack_rows(ctx->count_traversal ? 16 : stack_lds_of(ctx), lds_scene, closest), block, closest && !lds_scene) +
+  const bool dist = closest && !lds_scene;
+  const int depth = ctx->count_traversal ? 16 : dist ? closest_depth(stack_lds_of(ctx), block) : stack_lds_of(ctx);
+  const size_t lds = trace_lds_bytes(stack_rows(depth, lds_scene, dist), block, dist) +
                      (lds_scene ? (size_t)ctx->nnodes * sizeof(WideNode) + (size_t)ctx->ntri * sizeof(IsectTri) : 0);
-  const int by_lds = (int)std::min<size_t>(64, ctx->lds_per_cu / std::max<size_t>(1, lds));
+  const int by_lds = (int)std::min<size_t>(64, ctx->lds_per_cu / lds_granted(lds));
   return std::max(1, std::min({ctx->tuning.trace_blocks_per_cu, by_waves, by_lds}));
 }
 
@@ -2704,12 +2735,6 @@ int check_scene(gi_ctx *ctx, bool need_shading) {
         return fail(ctx, GI_ERR_STATE, "a material names a texture that was not uploaded (gi_upload_texture)");
   }
   return GI_OK;
-}
-
-// LDS bytes of a traversal block's stacks: `rows` entries per lane, lane
-// stride the next power of two >= block.
-size_t trace_lds_bytes(int rows, int block, bool dist) {
-  return stack_dist_bytes(rows, dist) + (size_t)rows * ((size_t)1 << lds_shift_for((uint32_t)block)) * sizeof(uint32_t);
 }
 
 InstScene inst_scene(const gi_ctx *ctx);
@@ -2789,7 +2814,7 @@ int launch_closest(gi_ctx *ctx, bool has_tmax, const QueueIn &Q, uint64_t n_boun
   int rc = trace_grid_for(ctx, n_bound, grid, block);
   if (rc) return rc;
   if (ts.max_grid > 0) grid = std::min(grid, ts.max_grid);
-  const int L = stack_lds_of(ctx);
+  const int L = stack_lds_of(ctx), LC = closest_depth(L, block);
   const bool I = instanced(ctx);
 #define GI_CL(T, II, LL) launch_closest_t<T, II, LL>(ctx, grid, block, Q, ro, rd, hits, ts)
 #define GI_CL_L(T, II) \
@@ -2797,8 +2822,8 @@ int launch_closest(gi_ctx *ctx, bool has_tmax, const QueueIn &Q, uint64_t n_boun
     launch_closest_t<T, II, 16, true>(ctx, grid, block, Q, ro, rd, hits, ts); \
   else if (!(II) && L == 16 && lds_scene_of(ctx)) \
     launch_closest_t<T, false, 16, false, true>(ctx, grid, block, Q, ro, rd, hits, ts); \
-  else if (L == 8) GI_CL(T, II, 8); \
-  else if (L == 32) GI_CL(T, II, 32); \
+  else if (LC == 8) GI_CL(T, II, 8); \
+  else if (LC == 32) GI_CL(T, II, 32); \
   else GI_CL(T, II, 16)
   if (has_tmax) {
     if (I) { GI_CL_L(true, true); } else { GI_CL_L(true, false); }

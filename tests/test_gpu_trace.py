@@ -150,6 +150,32 @@ def test_deep_stacks(stack_lds, block, instanced, oracle, gpu_ctx_factory):
         assert ((ctx.trace_any(o, d, t) != 0) == (ref["ref"] != 0xFFFFFFFF)).all()
 
 
+@pytest.mark.parametrize("block", [64, 128, 192])
+@pytest.mark.parametrize("stack_lds", [8, 16, 32])
+def test_stack_rows_of_smaller_blocks(stack_lds, block, oracle, gpu_ctx_factory):
+    """The stacks' LDS rows are as long as the block's lanes (the next power
+    of two): every block size, several waves per block, stacks within and
+    beyond the rows."""
+    n = 3000
+    tris = np.zeros(n, scenes.TRI)
+    z = (np.arange(n) * 0.01).astype(np.float32)
+    for k, (x, y) in zip("abc", [(-4, -4), (4, -4), (0, 5)]):
+        tris[k][:, 0], tris[k][:, 1], tris[k][:, 2] = x, y, z
+        tris["n" + k][:, 2] = 1
+    sc = scenes.Scene(tris, scenes.lambert((0.5, 0.5, 0.5)), None, None, None)
+    rng = np.random.default_rng(block + stack_lds)
+    m = 8000
+    o = np.stack([rng.uniform(-1, 1, m), rng.uniform(-1, 1, m), rng.uniform(-5, 35, m)], 1).astype(np.float32)
+    d = rng.normal(scale=[0.02, 0.02, 1.0], size=(m, 3)).astype(np.float32)
+    t = rng.choice(np.float32([FMAX, np.inf, 6.0, 0.004]), m)
+    ref = oracle.OracleScene(tris).trace_closest(o, d, t)
+    with gpu_ctx_factory() as ctx:
+        ctx.set_tuning(stack_lds=stack_lds, trace_block=block, trace_blocks_per_cu=24)
+        ctx.upload(sc, max_leaf=1)
+        assert (ctx.trace_closest(o, d, t) == ref).all()
+        assert ((ctx.trace_any(o, d, t) != 0) == (ref["ref"] != 0xFFFFFFFF)).all()
+
+
 @pytest.mark.parametrize("n", [1, 255, 16383, 16384, 16385])
 def test_host_trace_sizes(n, terrain, oracle, gpu_ctx_factory):
     """Calls on host arrays around the largest one that goes through pinned
