@@ -331,8 +331,11 @@ constexpr size_t kLdsSceneMaxBytes = 10240;
 // 256 lanes whatever the block, 12 instead of 24 blocks of 64 fitted a CU: 61
 // instead of 26 ms for the closest hits of a 3840x2160x8 frame of the
 // 4.2M-triangle scene; blocks of 128: 30.5 instead of 26.4 ms).
-// The kernels have no static LDS, so the dynamic LDS starts at address 0 and
-// entries are addressed by 32-bit offsets.  The global columns hold
+// Entries are addressed by 32-bit LDS addresses from 0 on, where the dynamic
+// LDS starts as long as these kernels have no static LDS: no __shared__
+// variable may come into them, and tests/test_kernel_resources.py looks at the
+// built kernels.  (The dynamic LDS's own address as the base is not folded
+// away by the compiler, and makes the kernels spill.)  The global columns hold
 // references only; entries from there are never dropped.
 struct StackEntry {
   uint32_t ref;
@@ -461,7 +464,7 @@ constexpr size_t trace_lds_bytes(int rows, int block, bool dist) {
 }
 
 template <int kRows, bool kDist>
-__device__ __forceinline__ Stack<kRows, kDist> make_stack(uint32_t *smem, uint32_t *gstack, uint32_t cap) {
+__device__ __forceinline__ Stack<kRows, kDist> make_stack(uint32_t *gstack, uint32_t cap) {
   const uint32_t shift = blockDim.x <= 1 ? 0u : 32u - (uint32_t)__clz((int)(blockDim.x - 1));
   using S = Stack<kRows, kDist>;
   const uint32_t rsh = shift + S::kUnit;
@@ -892,7 +895,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GI_TRACE_WA
     uint32_t n_tris) {
   extern __shared__ uint32_t smem[];
   constexpr bool kDist = !kLdsScene;
-  Stack<kRows, kDist> st = make_stack<kRows, kDist>(smem, gstack, stack_cap);
+  Stack<kRows, kDist> st = make_stack<kRows, kDist>(gstack, stack_cap);
   const float4 *lnodes = nullptr, *ltris = nullptr;
   stage_scene<kLdsScene>(smem, stack_words, wnodes, n_nodes, itris, n_tris, lnodes, ltris);
   trace_persistent<false, kInst, kRows, kCount, kLdsScene, kDist>(
@@ -920,7 +923,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GI_TRACE_WA
     uint32_t rec_stride, int32_t b, InstScene IS, unsigned long long *stats, uint32_t chunk_shift,
     uint32_t stack_words, uint32_t n_nodes, uint32_t n_tris) {
   extern __shared__ uint32_t smem[];
-  Stack<kRows, false> st = make_stack<kRows, false>(smem, gstack, stack_cap);
+  Stack<kRows, false> st = make_stack<kRows, false>(gstack, stack_cap);
   const float4 *lnodes = nullptr, *ltris = nullptr;
   stage_scene<kLdsScene>(smem, stack_words, wnodes, n_nodes, itris, n_tris, lnodes, ltris);
   trace_persistent<true, kInst, kRows, kCount, kLdsScene, false>(
