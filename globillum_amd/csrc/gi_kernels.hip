@@ -2107,7 +2107,7 @@ __global__ void k_fill_u32(uint32_t *__restrict__ p, uint32_t n, uint32_t v) {
 // aligned; blocks must be 256 threads.
 __global__ __launch_bounds__(256) void k_pack_image(const float4 *__restrict__ img, size_t first, uint32_t n,
                                                     float *__restrict__ out) {
-  __shared__ float s_rgb[768];
+  __shared__ __attribute__((aligned(16))) float s_rgb[768];  // read back as float4
   const uint32_t t = threadIdx.x;
   for (uint32_t p0 = blockIdx.x * 256u; p0 < n; p0 += gridDim.x * 256u) {
     if (p0 + t < n) {
