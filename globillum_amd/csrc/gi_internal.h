@@ -157,6 +157,24 @@ constexpr uint32_t kDoneRef = kLeafBit | kMaxLeafFirst;
 constexpr uint32_t kReturnRef = kLeafBit | (kMaxLeafFirst - 1);
 constexpr uint32_t kMaxInstances = kMaxLeafFirst - 2;
 
+// --------------------------------------------------------- ray queues ----
+// Consumers take spans or tiles j, j + stride, j + 2 stride, ... of a queue
+// of kShards segments: kShards consecutive ones of a segment, then as many of
+// the next (16 j's: kShards rows of every segment).  In the next 16 the
+// segments come in the same order, turned by one each time j passes a
+// multiple of 2^turn (any turn of at least 4 keeps the order complete: 16 j's
+// turn together).  With 2^turn the largest power of two that divides the
+// stride, a multiple of 16 for any full grid, a consumer's step turns by an
+// odd number: it meets the segments in turn, equally often.
+constexpr uint32_t kShardShift = 2, kShards = 1u << kShardShift;
+GI_HOST_DEVICE inline uint32_t queue_turn(uint32_t stride) {
+  const uint32_t t = (uint32_t)__builtin_ctz(stride);
+  return t > 2u * kShardShift ? t : 2u * kShardShift;
+}
+GI_HOST_DEVICE inline uint32_t queue_segment(uint32_t j, uint32_t turn) {
+  return ((j >> kShardShift) + (j >> turn)) & (kShards - 1u);
+}
+
 // ------------------------------------------------------------- Halton ----
 // Per-dimension constants of the scrambled radical inverse, laid out for
 // the device.  An index n < 2^32 is split, lowest digits first, into `full`

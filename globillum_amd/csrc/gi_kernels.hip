@@ -160,18 +160,20 @@ __device__ __forceinline__ float bitsf(uint32_t u) { return __uint_as_float(u); 
 // side: the 4.2M-triangle frame's any-hit kernel took 96 instead of 93 ms).  shift 0 is
 // a queue of one segment (a pass's path slots, the primitive entry points'
 // rays).
-constexpr uint32_t kShardShift = 2, kShards = 1u << kShardShift;
 constexpr uint32_t kCountStride = 16;  // 32-bit words between the counter pairs of two segments
 typedef __attribute__((address_space(4))) uint32_t const_u32;
+// The shading's turn (queue_segment): its blocks come and go as they finish,
+// so that no even share of the segments is needed.
+constexpr uint32_t kTileTurn = 11;
 struct QueueIn {
   const uint32_t *counts;  // n_k at counts[k * kCountStride], or null: one segment of n_host
   uint32_t n_host, shift, cap;
   // span or tile j: its segment, its row there, and the least row of the
-  // spans or tiles from j on.  The segment is turned by j / 2048, so that a
-  // wave that takes every 6144th span meets all segments: some are longer
-  // than others (unturned, the 291k-triangle frame's traversal took 2 % more)
-  __device__ __forceinline__ void locate(uint32_t j, uint32_t &k, uint32_t &row, uint32_t &least) const {
-    k = shift ? ((j >> kShardShift) + (j >> 11)) & (kShards - 1u) : 0u;
+  // spans or tiles from j on.  turn: queue_turn of the consumer's stride, so
+  // that it meets all segments: some are longer than others (unturned, the
+  // 291k-triangle frame's traversal took 2 % more)
+  __device__ __forceinline__ void locate(uint32_t j, uint32_t turn, uint32_t &k, uint32_t &row, uint32_t &least) const {
+    k = shift ? queue_segment(j, turn) : 0u;
     least = shift ? (j >> (2u * kShardShift)) << kShardShift : j;
     row = shift ? least | (j & (kShards - 1u)) : j;
   }
@@ -501,7 +503,7 @@ __device__ __forceinline__ void trace_persistent(QueueIn Q, uint32_t cs, const H
   uint32_t c_rays = 0, c_nodes = 0, c_tris = 0, c_inst = 0;
   const uint32_t lane = __lane_id();
   const uint64_t below = (1ull << lane) - 1ull;
-  const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+  const uint32_t waves = gridDim.x * (blockDim.x >> 6), turn = queue_turn(waves);
   const uint32_t chunk_n = 1u << cs;  // idle lanes a refill needs
   // span length 2^ss (wave-uniform): 16 spans per wave at least, 256 rays at most
   uint32_t total;
@@ -514,7 +516,7 @@ __device__ __forceinline__ void trace_persistent(QueueIn Q, uint32_t cs, const H
   const auto span_from = [&](uint32_t &j, uint32_t &b, uint32_t &e) {
     for (b = e = 0;; j += waves) {
       uint32_t k, row, least;
-      Q.locate(j, k, row, least);
+      Q.locate(j, turn, k, row, least);
       if (least >= rows) return;
       const uint32_t n = Q.size(k), off = row << ss;
       if (row < rows && off < n) {
@@ -1460,7 +1462,7 @@ __device__ __forceinline__ void shade_vertices(
   const uint32_t longest = Q.longest(total);
   for (uint32_t tile = blockIdx.x;; tile += gridDim.x) {
     uint32_t k, row, least;
-    Q.locate(tile, k, row, least);
+    Q.locate(tile, kTileTurn, k, row, least);
     if ((uint64_t)least * blockDim.x >= longest) break;
     const uint32_t off = row * blockDim.x, n_k = Q.size(k);
     if (off >= n_k) continue;  // this segment is shorter
@@ -1785,7 +1787,7 @@ __global__ __launch_bounds__(256) void k_shade_adjoint(int32_t b, QueueIn Q,
   const uint32_t longest = Q.longest(total);
   for (uint32_t tile = blockIdx.x;; tile += gridDim.x) {
     uint32_t k, row, least;
-    Q.locate(tile, k, row, least);
+    Q.locate(tile, kTileTurn, k, row, least);
     if ((uint64_t)least * blockDim.x >= longest) break;
     const uint32_t off = row * blockDim.x, n_k = Q.size(k);
     if (off >= n_k) continue;  // this segment is shorter
