@@ -126,19 +126,6 @@ struct HaltonDev {
   const HaltonDim *dims;
   const uint16_t *chunks;  // the chunk tables
 };
-// Chunk table entry c of dimension hd (the top chunk's table: c - P of the
-// entries past the full chunks').
-__device__ __forceinline__ uint16_t halton_entry(const HaltonDim &hd, const uint16_t *__restrict__ perms, uint32_t c) {
-  const bool top = c >= hd.P;
-  uint32_t x = top ? c - hd.P : c, v = 0;
-  const uint32_t m = top ? hd.mt : hd.m;
-  for (uint32_t i = 0; i < m; ++i) {  // least significant digit first
-    const uint32_t q = x / hd.prime;
-    v = v * hd.prime + perms[hd.perm_off + (x - q * hd.prime)];
-    x = q;
-  }
-  return (uint16_t)v;
-}
 // The chunk tables of dimension blockIdx.y.
 __global__ void __launch_bounds__(256) halton_fill(const HaltonDim *__restrict__ dims,
                                                    const uint16_t *__restrict__ perms,
@@ -149,54 +136,19 @@ __global__ void __launch_bounds__(256) halton_fill(const HaltonDim *__restrict__
 }
 
 typedef __attribute__((address_space(4))) HaltonDim HaltonDimConst;
-// Scrambled radical inverse of n in the prime base p of dimension dim: the
-// digits d_k (K of them) map to perm[d_k] and the infinitely many leading
-// zeros to perm[0], which is the exact rational
-//   A / B,  A = rev*(p-1) + perm[0],  B = p^K (p-1),  rev = sum perm[d_k] p^(K-1-k).
-// Leading zero digits may be counted as digits: each adds perm[0] to rev and
-// a factor p to p^K, which multiplies A and B by p and leaves A / B as it
-// is.  So every n < 2^32 is split into the same chunks of its dimension
-// (HaltonDim), and A, B < 2^32 p^2 are exact in FP64 (integers below 2^53).
-// The value is RN32(RN64(A / B)): with rB = RN(1/B) and q = RN(A rB), one
-// fused residual and one fused correction give the correctly rounded
-// quotient (Markstein, IBM J. Res. Dev. 34(1), 1990), three instructions in
-// place of the FP64 division's twenty.
-// Its quarter-rate integer products are the two of n / P (the top 32 bits
-// of the 96-bit n * magic; exact as the 64-bit mulhi) and one of the second
-// quotient: for q < 2^32 / P, floor(q / P) = mulhi(q, floor(2^32 / P) + 1),
-// since q times the multiplier's excess (<= P / 2^32) stays below 1 / P.
-// A sample's chunks are two of up to 65536 values and a top one (seven of up
-// to 1024, read from an LDS copy, before): the indices of a wave are mostly
-// consecutive, so its table reads fall into one or two lines (the low chunk)
-// or one entry (the others).  The shading kernels issue 22 % fewer vector
-// instructions with it and take 7.4 instead of 8.7 ms of the ~300k-triangle
-// frame and 85 instead of 97 ms of the 4.2M-triangle textured one; what
-// bounds them now is memory latency at 4 waves per SIMD.
+// halton_value of dimension dim.  A sample's chunks are two of up to 65536
+// values and a top one (seven of up to 1024, read from an LDS copy, before):
+// the indices of a wave are mostly consecutive, so its table reads fall into
+// one or two lines (the low chunk) or one entry (the others).  The shading
+// kernels issue 22 % fewer vector instructions with it and took 7.4 instead
+// of 8.7 ms of the ~300k-triangle frame and 85 instead of 97 ms of the
+// 4.2M-triangle textured one; what bounds them now is memory latency at 4
+// waves per SIMD.
 __device__ __forceinline__ float halton(uint32_t n, int dim, HaltonDev H) {
   // read through the constant address space: the dimension is the same for
   // every lane of a kernel's wave, so these are scalar loads (plain loads
   // would be vector loads, repeated after every store)
-  const HaltonDimConst &hd = ((const HaltonDimConst *)H.dims)[dim];
-  const uint16_t *tab = H.chunks + hd.off, *top = H.chunks + hd.top_off;
-  const uint32_t P = hd.P, mlo = (uint32_t)hd.magic, mhi = (uint32_t)(hd.magic >> 32);
-  // (n * mhi + hi32(n * mlo)) >> 32 = hi64(n * magic): the low word of
-  // n * mlo cannot carry into the top 32 bits of the 96-bit product
-  const uint32_t q0 = (uint32_t)(((uint64_t)n * mhi + __umulhi(n, mlo)) >> 32);
-  const uint32_t mq = mhi + 1u;  // floor(2^32 / P) + 1
-  const uint32_t q1 = __umulhi(q0, mq);
-  const uint32_t v0 = tab[n - __umul24(q0, P)], v1 = tab[q0 - __umul24(q1, P)];
-  uint32_t lo;
-  if (hd.full == 2) {  // uniform: one dimension per sample call
-    lo = top[q1];
-  } else {
-    const uint32_t q2 = __umulhi(q1, mq);
-    lo = __umul24(tab[q1 - __umul24(q2, P)], hd.Ptop) + top[q2];
-  }
-  const uint32_t hi = __umul24(v0, P) + v1;
-  const double A = fma((double)hi, hd.c_hi, fma((double)lo, hd.p1, hd.perm0d));
-  const double q = A * hd.rB;
-  const float f = (float)fma(fma(-q, hd.B, A), hd.rB, q);
-  return f >= 1.0f ? 0x1.fffffep-1f : f;
+  return halton_value(n, ((const HaltonDimConst *)H.dims)[dim], H.chunks);
 }
 
 // ---------------------------------------------------------- frames -------

@@ -198,6 +198,74 @@ struct HaltonDim {
 };
 static_assert(sizeof(HaltonDim) == 88, "halton dim layout");
 
+// Chunk table entry c of dimension hd (the top chunk's table: c - P of the
+// entries past the full chunks').
+GI_HOST_DEVICE inline uint16_t halton_entry(const HaltonDim &hd, const uint16_t *perms, uint32_t c) {
+  const bool top = c >= hd.P;
+  uint32_t x = top ? c - hd.P : c, v = 0;
+  const uint32_t m = top ? hd.mt : hd.m;
+  for (uint32_t i = 0; i < m; ++i) {  // least significant digit first
+    const uint32_t q = x / hd.prime;
+    v = v * hd.prime + perms[hd.perm_off + (x - q * hd.prime)];
+    x = q;
+  }
+  return (uint16_t)v;
+}
+// The product of two numbers below 2^24 (the hardware's full-rate one, which
+// drops higher bits).
+GI_HOST_DEVICE inline uint32_t mul24(uint32_t a, uint32_t b) { return (a & 0xffffffu) * (b & 0xffffffu); }
+GI_HOST_DEVICE inline uint32_t mul_hi(uint32_t a, uint32_t b) { return (uint32_t)(((uint64_t)a * b) >> 32); }
+
+// Scrambled radical inverse of n in the prime base p of a dimension: the
+// digits d_k (K of them) map to perm[d_k] and the infinitely many leading
+// zeros to perm[0], which is the exact rational
+//   A / B,  A = rev*(p-1) + perm[0],  B = p^K (p-1),  rev = sum perm[d_k] p^(K-1-k).
+// Leading zero digits may be counted as digits: each adds perm[0] to rev and
+// a factor p to p^K, which multiplies A and B by p and leaves A / B as it
+// is.  So every n < 2^32 is split into the same chunks of its dimension
+// (HaltonDim), and A, B < 2^53 are exact in FP64.
+//
+// The value is RN32(RN64(A / B)), the FP64 division and one rounding, from
+// rB = RN(1/B), q = RN(A rB) and one fused residual and correction
+// (Markstein, IBM J. Res. Dev. 34(1), 1990): three instructions in place of
+// the division's twenty.  q may be 1.5 ulp off, so RN64(A / B) itself is not
+// assured; the FP32 value is.  With every rounding at most 2^-53, what is
+// rounded last is x (1 + d), x = A / B, |d| <= 2^-104 (to first order).  The
+// two roundings give another FP32 value than from x only if a half-way point
+// of FP64 beside one of FP32, (j + 2^-29) / 2^(25+e) or (j - 2^-29) / 2^(25+e)
+// with j odd and 2^-e-1 < x < 2^-e, lies that near x: then B 2^-29 is within
+// 2^-26 of the integer |A 2^(25+e) - j B|, that is, B within 8 of a multiple
+// of 2^29.  No dimension's is (the nearest is 1.8 million away), but for
+// p = 2, whose B is a power of two and every step exact.
+//
+// The quarter-rate integer products are the two of n / P (the top 32 bits
+// of the 96-bit n * magic; exact as the 64-bit mulhi) and one of the second
+// quotient: for q < 2^32 / P, floor(q / P) = mul_hi(q, floor(2^32 / P) + 1),
+// since q times the multiplier's excess (<= P / 2^32) stays below 1 / P.
+// tests/csrc/sampler_check.cpp holds all these bounds for every dimension.
+template <class Dim> GI_HOST_DEVICE inline float halton_value(uint32_t n, Dim &hd, const uint16_t *chunks) {
+  const uint16_t *tab = chunks + hd.off, *top = chunks + hd.top_off;
+  const uint32_t P = hd.P, mlo = (uint32_t)hd.magic, mhi = (uint32_t)(hd.magic >> 32);
+  // (n * mhi + hi32(n * mlo)) >> 32 = hi64(n * magic): the low word of
+  // n * mlo cannot carry into the top 32 bits of the 96-bit product
+  const uint32_t q0 = (uint32_t)(((uint64_t)n * mhi + mul_hi(n, mlo)) >> 32);
+  const uint32_t mq = mhi + 1u;  // floor(2^32 / P) + 1
+  const uint32_t q1 = mul_hi(q0, mq);
+  const uint32_t v0 = tab[n - mul24(q0, P)], v1 = tab[q0 - mul24(q1, P)];
+  uint32_t lo;
+  if (hd.full == 2) {  // uniform: one dimension per sample call
+    lo = top[q1];
+  } else {
+    const uint32_t q2 = mul_hi(q1, mq);
+    lo = mul24(tab[q1 - mul24(q2, P)], hd.Ptop) + top[q2];
+  }
+  const uint32_t hi = mul24(v0, P) + v1;
+  const double A = __builtin_fma((double)hi, hd.c_hi, __builtin_fma((double)lo, hd.p1, hd.perm0d));
+  const double q = A * hd.rB;
+  const float f = (float)__builtin_fma(__builtin_fma(-q, hd.B, A), hd.rB, q);
+  return f >= 1.0f ? 0x1.fffffep-1f : f;
+}
+
 int32_t prime_of(int32_t dim);
 void halton_permutation(int32_t dim, uint32_t seed, uint16_t *perm);
 // The dimensions' constants, the digit permutations they index and the

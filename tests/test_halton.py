@@ -1,12 +1,17 @@
 """Halton sampler: the reference's radical inverse (src/util.cpp:22-32) and
 the scrambled extension, pinned by closed forms, the stratification
 property and an exact rational evaluation; product == oracle bit for bit."""
+import os
+import shutil
+import subprocess
 from fractions import Fraction
 
 import numpy as np
 import pytest
 
 from globillum_amd import _lib
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def test_radical_inverse_known_values(oracle):
@@ -90,75 +95,45 @@ def test_product_matches_oracle_bitwise(oracle):
     assert lib.gi_halton_prime(-1) == -1 and lib.gi_halton_prime(227) == 1439
 
 
-def test_every_dimension_needs_at_most_seven_chunks():
-    # the device splits an index n < 2^32 into at most 7 chunks of m digits,
-    # P = p^m <= 1024; that requires P^7 >= 2^32 for every dimension used
-    # (4 camera dimensions + 7 per vertex, 32 vertices)
-    lib = _lib.load()
-    for dim in range(4 + 7 * 32):
-        p = lib.gi_halton_prime(dim)
-        P = p
-        while P * p <= 1024:
-            P *= p
-        assert P ** 7 >= 2 ** 32, (dim, p, P)
+@pytest.fixture(scope="module")
+def sampler_check(tmp_path_factory):
+    hipcc = next((c for c in ("/opt/rocm/bin/hipcc", shutil.which("hipcc")) if c and os.path.exists(c)), None)
+    if hipcc is None:
+        pytest.skip("hipcc not found")
+    exe = str(tmp_path_factory.mktemp("sampler") / "sampler_check")
+    r = subprocess.run([hipcc, "-O2", "-std=c++17", "-ffp-contract=off", "-x", "c++", "-D__HIP_PLATFORM_AMD__",
+                        os.path.join(ROOT, "tests", "csrc", "sampler_check.cpp"),
+                        os.path.join(ROOT, "globillum_amd", "csrc", "bvh_build.cpp"), "-pthread", "-o", exe],
+                       capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return exe
 
 
-def test_sampler_tables_fit_the_lds_copy():
-    # ray generation copies the chunk tables of dimensions 0..3 into LDS, the
-    # untextured shading those of its vertex's 7 dimensions: 10240 entries
-    # hold every such window of a depth-32 render (the largest, dimensions
-    # 221..227, has 9959)
-    lib = _lib.load()
-    sizes = []
-    for dim in range(4 + 7 * 32):
-        p = lib.gi_halton_prime(dim)
-        P = p
-        while P * p <= 1024:
-            P *= p
-        sizes.append(P)
-    windows = [sum(sizes[0:4])] + [sum(sizes[d:d + 7]) for d in range(4, 4 + 7 * 32, 7)]
-    assert windows[0] == 2721 and max(windows) == 9959 and max(windows) <= 10240
+@pytest.mark.parametrize("seed", [0, 7, 2 ** 32 - 1])
+def test_kernel_sampler_on_the_host(sampler_check, seed):
+    """The kernels' sampler function and tables, compiled for the host
+    (tests/csrc/sampler_check.cpp): the bounds they rest on hold for every
+    dimension of a depth-32 render, and the values are the digit loop's at the
+    chunks' boundaries, the ends of the range and 20000 random indices each."""
+    r = subprocess.run([sampler_check, str(seed), "20000"], capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0 and "bad: bounds 0 edges 0 random 0" in r.stdout, r.stdout[-2000:]
 
 
-def test_fixed_chunk_count_keeps_the_rational(oracle):
-    # the kernels split every index n < 2^32 into the same kmax chunks of its
-    # dimension (the least K with P^K >= 2^32), zero chunks above the leading
-    # one included: each zero chunk multiplies A and B by P, so A / B is the
-    # digit loop's rational, and A, B stay below 2^53 (exact in FP64) for
-    # every dimension of a depth-32 render
-    from fractions import Fraction
-
-    lib = _lib.load()
-    rng = np.random.default_rng(5)
-    seed = 7
-    for dim in range(4 + 7 * 32):
-        p = lib.gi_halton_prime(dim)
-        P, m = p, 1
-        while P * p <= 1024:
-            P *= p
-            m += 1
-        kmax, pk = 0, 1
-        while pk < 2 ** 32:
-            pk *= P
-            kmax += 1
-        assert pk * p < 2 ** 53, (dim, p, P, kmax)
-        perm = oracle.halton_perm(dim, seed).astype(np.int64)
-        for n in [0, 1, P - 1, P, P * P, 2 ** 32 - 1] + [int(x) for x in rng.integers(0, 2 ** 32, 4)]:
-            rev, pk_d, x = 0, 1, n
-            while x:
-                rev = rev * p + int(perm[x % p])
-                pk_d *= p
-                x //= p
-            exact = Fraction(rev * (p - 1) + int(perm[0]), pk_d * (p - 1))
+@pytest.mark.parametrize("dim", [0, 1, 2, 53, 54, 227])
+def test_digit_split_keeps_the_rational(oracle, dim):
+    """Counting leading zeros as digits, up to a fixed number of them, leaves
+    A / B as it is (the kernels' splits always count as many)."""
+    p = oracle.prime(dim)
+    perm = oracle.halton_perm(dim, 7).astype(np.int64)
+    rng = np.random.default_rng(dim)
+    for n in [0, 1, p - 1, p, 2 ** 32 - 1] + [int(x) for x in rng.integers(0, 2 ** 32, 8)]:
+        exact = _exact(n, p, perm)
+        k = 0
+        while p ** k < 2 ** 32:
+            k += 1
+        for digits in range(k, k + 3):
             rev, x = 0, n
-            for _ in range(kmax):
-                c = x % P
-                x //= P
-                v, y = 0, c
-                for _ in range(m):  # the chunk table entry: least significant digit first
-                    v = v * p + int(perm[y % p])
-                    y //= p
-                rev = rev * P + v
-            assert x == 0
-            A, B = rev * (p - 1) + int(perm[0]), pk * (p - 1)
-            assert A < 2 ** 53 and B < 2 ** 53 and Fraction(A, B) == exact, (dim, n)
+            for _ in range(digits):
+                rev = rev * p + int(perm[x % p])
+                x //= p
+            assert x == 0 and Fraction(rev * (p - 1) + int(perm[0]), p ** digits * (p - 1)) == exact
