@@ -84,7 +84,9 @@ struct Builder {
       for (int k = 0; k < 3; ++k) cen[3 * i + k] = 0.5f * (tbox[i].lo[k] + tbox[i].hi[k]);
     }
   }
-  // over the boxes of triangles, as the first constructor makes them
+  // over the boxes of triangles as the first constructor makes them, and so
+  // taken as they are: an axis on which a triangle has NaN corners only has
+  // lo above hi, which growing a box by lo and hi (below) would turn round
   Builder(const TriBox *t, int64_t n, int32_t ml, std::vector<uint32_t> &p, std::vector<Bvh2Node> &nd)
       : tris(nullptr), tbox(n), cen(3 * n), perm(p), nodes(nd), max_leaf(ml) {
     for (int64_t i = 0; i < n; ++i)

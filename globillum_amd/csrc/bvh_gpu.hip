@@ -1251,10 +1251,23 @@ __global__ void k_sah_last(uint32_t *__restrict__ ne, uint32_t nodes) {
     hipError_t e_ = (x);                                              \
     if (e_ != hipSuccess) {                                           \
       err = std::string(#x) + ": " + hipGetErrorString(e_);           \
-      for (void *p : mem) (void)hipFree(p);                           \
       return false;                                                   \
     }                                                                 \
   } while (0)
+
+// Device allocations that last as long as this.
+struct DeviceBlocks {
+  std::vector<void *> blocks;
+  ~DeviceBlocks() {
+    for (void *p : blocks) (void)hipFree(p);
+  }
+  void *get(size_t bytes) {
+    void *p = nullptr;
+    if (hipMalloc(&p, std::max<size_t>(bytes, 16)) != hipSuccess) return nullptr;
+    blocks.push_back(p);
+    return p;
+  }
+};
 
 // Places arrays one after another (256-byte aligned) in one block: carved
 // once without a block for its size, then again in the block.
@@ -1349,13 +1362,8 @@ static bool emit_wide(hipStream_t s, const CollapseArgs &A, int32_t root, WideNo
 static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_t n, int max_leaf, int W,
                              WideNode *nodes, float4 *itris, const std::function<void *(size_t)> &scratch, LbvhResult &res,
                              std::string &err) {
-  std::vector<void *> mem;
-  auto alloc = [&](size_t bytes) -> void * {
-    void *p = nullptr;
-    if (hipMalloc(&p, std::max<size_t>(bytes, 16)) != hipSuccess) return nullptr;
-    mem.push_back(p);
-    return p;
-  };
+  DeviceBlocks mem;  // a segmented sort's buffers
+  const auto alloc = [&](size_t bytes) { return mem.get(bytes); };
   const size_t nn = 2 * (size_t)n;  // binary nodes: at most 2n - 1
   // a level lists the children of split nodes (more than max_leaf triangles each)
   const size_t lcap = std::min<size_t>(n, 2 * ((size_t)n / (max_leaf + 1)) + 2);
@@ -1432,7 +1440,6 @@ static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, 
     if (count == 0) break;
     if (depth > kSahMaxDepth + 64 || count > lcap) {
       err = "device bvh: SAH build did not terminate";
-      for (void *q : mem) (void)hipFree(q);
       return false;
     }
     const int32_t *list = lvl + off[off.size() - 2];
@@ -1468,7 +1475,6 @@ static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, 
     if (splits == 0) break;  // every node of the level is a leaf
     if ((size_t)nodes_made + 2 * (size_t)splits > nn - 1 || 2 * (size_t)splits > lcap) {
       err = "device bvh: SAH node count exceeded";
-      for (void *q : mem) (void)hipFree(q);
       return false;
     }
     hipLaunchKernelGGL(k_sah_children, dim3(blocks(count)), dim3(kBlock), 0, s, S, count, pre, nodes_made, flags,
@@ -1481,7 +1487,6 @@ static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, 
       vals2 = (uint32_t *)alloc(4 * (size_t)n);
       if (!keys || !keys2 || !vals || !vals2) {
         err = "device bvh: out of device memory (median sort)";
-        for (void *q : mem) (void)hipFree(q);
         return false;
       }
     }
@@ -1496,7 +1501,6 @@ static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, 
         sort_bytes = need;
         if (!sort_temp) {
           err = "device bvh: out of device memory (median sort)";
-          for (void *q : mem) (void)hipFree(q);
           return false;
         }
       }
@@ -1528,14 +1532,12 @@ static bool device_sah_build(hipStream_t s, const float4 *tri, uint32_t stride, 
     ok = emit_wide(s, A, 0, nodes, front, cnt, res, err);
   }
   res.rounds = (int32_t)(off.size() - 2);  // binary levels below the root
-  for (void *q : mem) (void)hipFree(q);
   return ok;
 }
 
 bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_t n, const float clo[3],
                       const float chi[3], int max_leaf, DeviceBvhMethod method, int radius, int width, WideNode *nodes,
                       float4 *itris, const std::function<void *(size_t)> &scratch, LbvhResult &res, std::string &err) {
-  std::vector<void *> mem;  // none: the scratch block holds everything
   if (n == 0 || max_leaf < 1 || max_leaf > kMaxLeafTris) {
     err = "device bvh: n > 0 and 1 <= max_leaf <= 15 required";
     return false;
@@ -1649,7 +1651,6 @@ bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_
         GI_CK(hipStreamSynchronize(s));
         if (nc > ni - off.back()) {
           err = "device bvh: radix tree levels exceed its node count";
-          for (void *q : mem) (void)hipFree(q);
           return false;
         }
         off.push_back(off.back() + nc);
@@ -1683,7 +1684,6 @@ bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_
     while (bound > 1) {
       if ((size_t)rounds > (size_t)n) {  // the round log holds n + kRoundsPerSync + 1 entries
         err = "device bvh: PLOC clustering stalled (too many rounds)";
-        for (void *q : mem) (void)hipFree(q);
         return false;
       }
       for (int r = 0; r < kRoundsPerSync; ++r) {
@@ -1706,7 +1706,6 @@ bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_
       // every round merges at least the globally closest pair
       if (tot[0] >= bound || tot[0] == 0 || tot[0] + tot[1] != n) {
         err = "device bvh: PLOC clustering stalled (non-finite vertex coordinates?)";
-        for (void *q : mem) (void)hipFree(q);
         return false;
       }
       bound = tot[0];
@@ -1730,7 +1729,6 @@ bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_
       for (int r = 0; r < rounds; ++r) {
         if (rn[r + 1] < rn[r] || rn[r + 1] > ni) {
           err = "device bvh: PLOC round log out of order";
-          for (void *q : mem) (void)hipFree(q);
           return false;
         }
         const uint32_t c = rn[r + 1] - rn[r];
@@ -1746,7 +1744,6 @@ bool device_bvh_build(hipStream_t s, const float4 *tri, uint32_t stride, uint32_
   // root is node 0 and PLOC's the last merge, n - 2
   const bool ok = n == 1 ? emit_single_leaf(s, leafbox, 1u, nodes, res, err)
                          : emit_wide(s, A, ploc ? (int32_t)(n - 2) : 0, nodes, front, cnt, res, err);
-  for (void *q : mem) (void)hipFree(q);
   return ok;
 }
 

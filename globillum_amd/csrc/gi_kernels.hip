@@ -2321,10 +2321,13 @@ constexpr int kStageSlots = 8;
 constexpr size_t kStageBytes = (size_t)768 << 10;
 constexpr uint32_t kStagePixels = (uint32_t)(kStageBytes / 12);
 // The staging memory of the read-backs under way: a read-back takes a block
-// (6 MB) and gives it back when its copies have landed.  Pinning a block
-// takes 0.9 ms, as long as reading a 1280x720 image, so up to two free
+// (6 MB) and gives it back when its copies have landed.  A new block costs
+// the allocation (0.08 to 0.3 ms) and the first touch of the pages in use
+// (up to 0.8 ms), as long as reading a 1280x720 image, so up to two free
 // blocks are kept for the process's next read-backs, on any thread and
-// device, until its last context is destroyed.
+// device, until its last context is destroyed.  (Leaving a context's first
+// small image to a pageable copy instead was tried: 9.0 against 1.1 ms for a
+// process's first 512x512 image.)
 std::mutex g_stage_mu;
 constexpr int kStageKept = 2;
 uint8_t *g_stage_free[kStageKept];
@@ -4162,8 +4165,11 @@ int gi_trace_closest_device_noalloc(gi_ctx *ctx, const float *d_orig, const floa
 namespace {
 // Host-array traces of at most this many rays go through a pinned block:
 // the kernels read the rays and write the results there, and the call waits
-// once.  Larger ones copy (a copy engine moves pageable arrays faster than
-// this thread moves them into the block).
+// once.  Larger ones copy.  The line is not where the two cross: closest
+// hits of 1024, 16384, 32768 and 131072 rays through 35k triangles take
+// 72, 97, 124 and 320 us by the block and 170, 162, 174 and 405 us by
+// copies (34 triangles: 39, 64, 91 and 290 against 139, 124, 135 and 362
+// us), and a block holds 142000 rays.
 constexpr int64_t kPinnedTraceRays = 16384;
 static_assert((28 + 16) * kPinnedTraceRays + 64 <= (int64_t)(kStageSlots * kStageBytes), "the block holds a call's rays");
 
