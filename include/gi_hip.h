@@ -194,7 +194,10 @@ typedef struct {
   int32_t trace_blocks_per_cu;
   int32_t shade_block;
   int32_t samples_per_pass;
-  int32_t stack_lds;        /* traversal stack entries per lane in LDS: 8, 16 or 32 */
+  int32_t stack_lds;        /* depth of the traversal stack's LDS part: 8, 16 or 32
+                               (the rows of entries per lane that a depth stands for
+                               are 12, 16 and 32 for closest hits and 12, 20 and 32
+                               for any hits; deeper entries lie in device memory) */
   int32_t target_slots;     /* paths in flight per pass, in units of 2^20: 0..256,
                                0 = 128 (about 30 GB of path state with textures) */
   int32_t node_width;       /* child slots the collapse fills per BVH node: 2, 3 or 4

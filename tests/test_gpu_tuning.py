@@ -4,7 +4,7 @@ or on the traversal kernels' refill threshold (8..64 lanes); narrower nodes
 mean more node visits; invalid values and a node-width change under placed
 instances are refused; the autotuner returns a setting from its space,
 leaves it applied, and the image rendered with it is the default one.  A
-scene small enough for the traversal kernels' LDS copy (at most 16 KB of
+scene small enough for the traversal kernels' LDS copy (at most 10 KB of
 nodes and triangles; LDS stack depth 16) renders and traces exactly as
 through the global-memory kernels (stack depth 8 or 32)."""
 import numpy as np
