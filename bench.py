@@ -276,14 +276,26 @@ def b_ray(per_ray: dict, kind: str) -> float:
     return 32 + 16 + 32 * per_ray[f"box_{kind}"] + 40 * per_ray[f"tri_{kind}"]
 
 
+def requested_per_ray(ts: dict, kind: str) -> float:
+    """Bytes a ray of the traversal asks for (kind closest or any): the ray, its
+    result, a 128-byte line per node visited, 48 bytes per triangle tested."""
+    n = max(1, ts[f"{kind}_rays"])
+    return 32 + 16 + (128 * ts[f"{kind}_nodes"] + 48 * ts[f"{kind}_triangles"]) / n
+
+
 def roofline_entry(kernel: str, bytes_per_launch: float, ms_total: float, launches: int, bw: dict | None,
-                   cached: bool, traffic: dict | None = None, unit_bytes: dict | None = None) -> dict:
+                   cached: bool, traffic: dict | None = None, unit_bytes: dict | None = None,
+                   requested: float | None = None) -> dict:
     """One kernel's roofline record.  cached: the kernel's reads are mostly
     served by the caches (the traversal kernels: the measured HBM traffic is
     a fraction of the algorithmic bytes), so its bound is the measured L2
     read bandwidth; otherwise (and without that measurement) the 8 TB/s HBM
     peak.  The HBM figures stay beside: the algorithmic bytes over the HBM
-    peak and the measured traffic's rate over the HBM peak."""
+    peak and the measured traffic's rate over the HBM peak.  achieved and
+    frac are an equivalent rate where the kernel asks for fewer bytes than the
+    reference's traversal rules count; requested (bytes per launch, by the
+    counting build) gives the rate it draws, as requested_gbs and
+    frac_requested."""
     avg_s = ms_total / max(1, launches) / 1e3
     achieved = bytes_per_launch / avg_s / 1e9 if avg_s > 0 else 0.0
     if cached and bw:
@@ -296,6 +308,9 @@ def roofline_entry(kernel: str, bytes_per_launch: float, ms_total: float, launch
          "algorithmic_bytes_per_launch": round(bytes_per_launch)}
     if bound != "hbm":
         e["frac_of_hbm_peak_algorithmic"] = round(achieved / HBM_PEAK_GBS, 4)
+    if requested and avg_s > 0:
+        e["requested_gbs"] = round(requested / avg_s / 1e9, 1)
+        e["frac_requested"] = round(requested / avg_s / 1e9 / peak, 4)
     if unit_bytes:
         e.update(unit_bytes)
     if traffic:
@@ -412,24 +427,26 @@ def headline(a, threads, host, traffic, bw):
         rc = tot["rays_closest"] / L
         rs = tot["rays_shadow"] / L
         tr = traffic or {}
+        req = {k: requested_per_ray(ts, k) for k in ("closest", "any")}
         roof = roofline_entry("k_trace_closest (two-level)", rc * b_ray(per_ray, "closest"), tot["ms_trace_closest"],
-                              L, bw, True, traffic=tr.get("large.trace_closest"),
+                              L, bw, True, traffic=tr.get("large.trace_closest"), requested=rc * req["closest"],
                               unit_bytes={"algorithmic_bytes_per_ray": round(b_ray(per_ray, "closest"), 1),
                                           "rays_per_launch": round(rc)})
         roof["others"] = {
             "k_trace_any": roofline_entry("k_trace_any (two-level)", rs * b_ray(per_ray, "shadow"),
                                           tot["ms_trace_any"], L, bw, True, traffic=tr.get("large.trace_any"),
+                                          requested=rs * req["any"],
                                           unit_bytes={"algorithmic_bytes_per_ray": round(b_ray(per_ray, "shadow"), 1),
                                                       "rays_per_launch": round(rs)}),
             "k_shade_tex": roofline_entry("k_shade_tex", rc * B_VERTEX_TEX, tot["ms_shade"], L, bw, False,
                                           traffic=tr.get("large.shade"),
                                           unit_bytes={"algorithmic_bytes_per_vertex": B_VERTEX_TEX,
                                                       "vertices_per_launch": round(rc)})}
-        req = 32 + 16 + (128 * ts["closest_nodes"] + 48 * ts["closest_triangles"]) / max(1, ts["closest_rays"])
         roof["wide_traversal"] = {"nodes_per_ray": round(ts["closest_nodes"] / max(1, ts["closest_rays"]), 3),
                                   "triangles_per_ray": round(ts["closest_triangles"] / max(1, ts["closest_rays"]), 3),
                                   "instances_per_ray": round(ts["closest_instances"] / max(1, ts["closest_rays"]), 3),
-                                  "requested_bytes_per_ray": round(req, 1)}
+                                  "requested_bytes_per_ray": round(req["closest"], 1),
+                                  "requested_bytes_per_shadow_ray": round(req["any"], 1)}
         if bw:
             roof["measured_read_gbs"] = bw
     rays = tot["rays_closest"] + tot["rays_shadow"]
@@ -517,18 +534,21 @@ def plain_leg(steps: int, threads: int, host, traffic, bw, with_cpu: bool):
         rc, rs = tot["rays_closest"] / L, tot["rays_shadow"] / L
         tr = traffic or {}
         roof = {}
-        for name, nbytes, ms, tk, ub in (
+        req = {k: requested_per_ray(ts, k) for k in ("closest", "any")}
+        for name, nbytes, ms, tk, ub, rq in (
                 ("k_trace_closest", rc * b_ray(per_ray, "closest"), tot["ms_trace_closest"], "plain.trace_closest",
-                 {"algorithmic_bytes_per_ray": round(b_ray(per_ray, "closest"), 1)}),
+                 {"algorithmic_bytes_per_ray": round(b_ray(per_ray, "closest"), 1)}, rc * req["closest"]),
                 ("k_trace_any", rs * b_ray(per_ray, "shadow"), tot["ms_trace_any"], "plain.trace_any",
-                 {"algorithmic_bytes_per_ray": round(b_ray(per_ray, "shadow"), 1)}),
-                ("k_shade", rc * B_VERTEX, tot["ms_shade"], "plain.shade", {"algorithmic_bytes_per_vertex": B_VERTEX})):
-            roof[name] = roofline_entry(name, nbytes, ms, L, bw, name != "k_shade", traffic=tr.get(tk), unit_bytes=ub)
-        req = 32 + 16 + (128 * ts["closest_nodes"] + 48 * ts["closest_triangles"]) / max(1, ts["closest_rays"])
+                 {"algorithmic_bytes_per_ray": round(b_ray(per_ray, "shadow"), 1)}, rs * req["any"]),
+                ("k_shade", rc * B_VERTEX, tot["ms_shade"], "plain.shade",
+                 {"algorithmic_bytes_per_vertex": B_VERTEX}, None)):
+            roof[name] = roofline_entry(name, nbytes, ms, L, bw, name != "k_shade", traffic=tr.get(tk), unit_bytes=ub,
+                                        requested=rq)
         roof["k_trace_closest"]["wide_traversal"] = {
             "nodes_per_ray": round(ts["closest_nodes"] / max(1, ts["closest_rays"]), 3),
             "triangles_per_ray": round(ts["closest_triangles"] / max(1, ts["closest_rays"]), 3),
-            "requested_bytes_per_ray": round(req, 1)}
+            "requested_bytes_per_ray": round(req["closest"], 1),
+            "requested_bytes_per_shadow_ray": round(req["any"], 1)}
         out["roofline"] = roof
     log(f"plain leg: {out['mrays_per_s']} Mrays/s")
     return out
