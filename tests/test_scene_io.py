@@ -149,7 +149,8 @@ def test_errors(objdir, tmp_path):
         scene_io.read_pbrdf(str(p))
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference asset files not present")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REF, "plainSphere.obj")),
+                    reason="reference asset files not present")
 def test_reference_assets():
     tris, mats, names = _compare([os.path.join(REF, "plainSphere.obj")], pbrdf_dir=os.path.join(REF, "materials"))
     # 720 triangles on the unit sphere; usemtl "default" is not in its MTL -> fallback
