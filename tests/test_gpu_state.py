@@ -251,10 +251,10 @@ def test_image_readback_sizes(w, h, oracle, gpu_ctx_factory):
 
 
 @pytest.mark.parametrize("builder", ["host", "sah", "device", "ploc"])
-@pytest.mark.parametrize("n", [1, 127, 128, 129, 3000, 131_200])
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 2175, 2176, 2177, 3000, 131_200])
 def test_triangle_upload_sizes(n, builder, oracle, gpu_ctx_factory):
-    """Triangle tables around the upload's blocks (128 triangles, 1024
-    blocks), each replacing the one before: hits, and an image whose ray
+    """Triangle tables converted by the host (up to 2048) and around the
+    device conversion's blocks (128 triangles, 1024 blocks), each replacing the one before: hits, and an image whose ray
     offsets come from the scene's bounds, are the oracle's."""
     def soup(n, seed):
         rng = np.random.default_rng(seed)
@@ -280,3 +280,41 @@ def test_triangle_upload_sizes(n, builder, oracle, gpu_ctx_factory):
         d = rng.normal(size=(2000, 3)).astype(np.float32)
         t = np.full(2000, np.finfo(np.float32).max, np.float32)
         assert (ctx.trace_closest(o, d, t) == osc.trace_closest(o, d, t)).all()
+
+
+@pytest.mark.parametrize("builder", ["host", "sah"])
+@pytest.mark.parametrize("n", [1, 2, 127, 2048])
+def test_host_and_device_conversion_agree(n, builder, gpu_ctx_factory):
+    """Small scenes (up to 2048 triangles) are converted by the host, larger
+    ones on the device: n triangles, alone and among 2049 whose others are
+    points inside the scene (hit by nothing), give the same image -- its ray
+    offsets come from the bounds -- and the same hits; with the host builder
+    also where corners are NaN, which bounds pass over."""
+    rng = np.random.default_rng(n)
+    t = np.zeros(n, scenes.TRI)
+    c = rng.uniform(-5, 5, (n, 3))
+    for k in "abc":
+        t[k] = c + rng.normal(scale=0.5, size=(n, 3))
+        t["n" + k] = rng.normal(size=3)
+        t["t" + k] = rng.uniform(size=(n, 2))
+    t["material_index"] = rng.integers(0, 3, n)
+    if builder == "host" and n > 2:
+        t["b"][n // 2, 1] = np.nan
+        t["a"][n // 3, 0] = np.nan
+    points = np.zeros(2049 - n, scenes.TRI)
+    for k in "abc":
+        points[k] = t["c"][0]
+        points["n" + k] = t["n" + k][0]
+    points["material_index"] = t["material_index"][0]
+    mats = np.concatenate([scenes.lambert(rng.uniform(0.2, 0.8, 3)) for _ in range(3)])
+    light = scenes.make_light((0, 9, 0), (0, -1, 0), (30, 30, 30), 4, 4)
+    view = scenes.make_view((0, 0, -14), (0, 0, 0), (0, 1, 0), 50.0, 40, 30, 2)
+    o = rng.uniform(-6, 6, (3000, 3)).astype(np.float32)
+    d = rng.normal(size=(3000, 3)).astype(np.float32)
+    m = np.full(3000, np.finfo(np.float32).max, np.float32)
+    out = []
+    with gpu_ctx_factory() as ctx:
+        for tris in (t, np.concatenate([t, points])):
+            ctx.upload(scenes.Scene(tris, mats, light, view, scenes.make_opts(3)), builder=builder)
+            out.append((ctx.render().image(0).copy(), ctx.trace_closest(o, d, m)))
+    assert np.array_equal(out[0][0], out[1][0]) and (out[0][1] == out[1][1]).all()
