@@ -324,9 +324,9 @@ constexpr size_t kLdsSceneMaxBytes = 10240;
 // of its box, so that it can be dropped without a node visit once a hit
 // nearer than it is known.  Of the distance only the upper 16 bits are kept
 // in LDS (rounded towards zero: nothing is dropped too early): 6 bytes an
-// entry, 16 rows at 6 waves per SIMD.  8-byte entries leave 13
-// rows: 2 % faster on a 291k-triangle tree and 1.3 % slower on the 4.2M-
-// triangle two-level one, whose stacks run past 13 rows more often.
+// entry, 16 rows at 6 waves per SIMD.  8-byte entries leave 13 rows: 2 %
+// faster on a 291k-triangle tree and 1.3 % slower on the 4.2M-triangle
+// two-level one, whose stacks run past 13 rows more often.
 // LDS layout: the distances, then the references, both interleaved by lane
 // (no bank conflicts) in rows of the next power of two of the block's lanes,
 // so that a block of any size takes 6 bytes an entry and lane (with rows for
